@@ -15,7 +15,7 @@ one GPU.  Per-stage device times come from HIP events that the library
 records on its stream between the stages of every timed realization (no host
 synchronisation inside the timed region).  `roofline` covers the dominant
 stage: algorithmic bytes per launch / its average launch time (the pit
-fill is two kernels, k_pf_persistent and k_pf_resident).  Unless
+fill is two kernels, k_pf_start and k_pf_fill).  Unless
 --no-traffic, `traffic` is the HBM bytes per launch of those kernels from two
 rocprofv3 counter passes (FETCH_SIZE, then WRITE_SIZE) over a short probe
 run (`--probe`), scaled by what the same counters read for an elementwise
@@ -66,7 +66,7 @@ STAGE_NAMES = ["random_field", "convolution", "realistic_burn", "pit_fill", "flo
 # kernel ends at once when the first kernel converged alone).
 STAGE_KERNEL = {
     "random_field": ("k_random_field",), "realistic_burn": ("k_realistic_burn_quant",),
-    "pit_fill": ("k_pf_persistent", "k_pf_resident"),
+    "pit_fill": ("k_pf_start", "k_pf_fill"),
     "flow_routing": ("k_fr_d8", "k_fr_persistent", "k_fr_pick"),
     "flow_tracing": ("k_tr_tiles", "k_tr_jump", "k_tr_exits"), "border": ("k_border",),
 }

@@ -43,7 +43,7 @@ int alloc(T** p, size_t count) {
 }
 
 void free_all(Context* c) {
-    void* ptrs[] = {c->d_mark, c->d_mark_pf, c->d_topen, c->d_tcost, c->d_rows, c->d_work3, c->d_ctrl, c->d_bar, c->d_scal, c->d_bmm, c->d_filter,
+    void* ptrs[] = {c->d_mark, c->d_xb, c->d_pfmask, c->d_pfinfo, c->d_rows, c->d_work3, c->d_ctrl, c->d_bar, c->d_scal, c->d_bmm, c->d_filter,
                     c->d_sflags, c->d_slabel, c->d_off, c->d_factor, c->d_a, c->d_b, c->d_z,
                     c->d_w, c->d_st, c->d_fd, c->d_dist, c->d_lab, c->d_ptr, c->d_bent,
                     c->d_lr_col, c->d_lr_row, c->d_lr_planes};
@@ -235,10 +235,10 @@ int cageo_context_create(cageo_context** out, int W, int H, void* stream) {
         if (st == CAGEO_OK) st = s;
     };
     A(cageo::alloc(&c->d_mark, c->ntiles));
-    A(cageo::alloc(&c->d_mark_pf, c->ntiles));
     A(cageo::alloc(&c->d_rows, 4 * (size_t)c->ntiles));
-    A(cageo::alloc(&c->d_topen, c->ntiles));
-    A(cageo::alloc(&c->d_tcost, c->ntiles));
+    A(cageo::alloc(&c->d_xb, 768 * (size_t)c->ntiles));
+    A(cageo::alloc(&c->d_pfmask, cageo::TILE_THREADS * (size_t)c->ntiles));
+    A(cageo::alloc(&c->d_pfinfo, c->ntiles));
     A(cageo::alloc(&c->d_work3, 7 * (size_t)c->ntiles));
     A(cageo::alloc(&c->d_ctrl, cageo::CTL_WORDS));
     A(cageo::alloc(&c->d_bar, cageo::BAR_WORDS));
@@ -281,7 +281,6 @@ int cageo_context_create(cageo_context** out, int W, int H, void* stream) {
     }
     if (st == CAGEO_OK &&
         (hipMemsetAsync(c->d_mark, 0, (size_t)c->ntiles * sizeof(uint32_t), c->stream) != hipSuccess ||
-         hipMemsetAsync(c->d_mark_pf, 0, (size_t)c->ntiles * sizeof(uint32_t), c->stream) != hipSuccess ||
          hipMemsetAsync(c->d_ctrl, 0, cageo::CTL_WORDS * sizeof(uint32_t), c->stream) != hipSuccess ||
          hipMemsetAsync(c->d_bar, 0, cageo::BAR_WORDS * sizeof(uint32_t), c->stream) != hipSuccess ||
          hipMemsetAsync(c->d_scal, 0, cageo::SC_NSLOTS * sizeof(uint32_t), c->stream) != hipSuccess ||
@@ -529,7 +528,7 @@ int cageo_realization_from_noise(cageo_context* ctx, float* d_noise, float* d_mc
 int cageo_iteration_counts(cageo_context* ctx, int32_t* out) {
     if (!ctx || !out) return CAGEO_ERR_ARG;
     Context* c = &ctx->c;
-    uint32_t h[cageo::CTL_WORDS];
+    uint32_t h[cageo::CTL_PF_COUNTS];  // the words before the pit fill's counters
     CAGEO_HIP_TRY(hipMemcpyAsync(h, c->d_ctrl, sizeof(h), hipMemcpyDeviceToHost, c->stream));
     CAGEO_HIP_TRY(hipStreamSynchronize(c->stream));
     out[0] = (int32_t)h[cageo::CTL_ROUNDS];

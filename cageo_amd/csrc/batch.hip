@@ -212,15 +212,13 @@ int multi_setup(MultiState* m, Context* const* ctxs, int nr) {
     };
     A(dev_alloc(&m->d_base, (size_t)nr + 1));
     A(dev_alloc(&m->d_bmap, (size_t)m->total));
-    A(dev_alloc(&m->d_rinfo, (size_t)nr));
     A(dev_alloc(&m->d_work, 7 * (size_t)m->total));
-    A(dev_alloc(&m->d_mark_pf, (size_t)m->total));
+    A(dev_alloc(&m->d_xb, 768 * (size_t)m->total));
+    A(dev_alloc(&m->d_pfmask, TILE_THREADS * (size_t)m->total));
+    A(dev_alloc(&m->d_pfinfo, (size_t)m->total));
     A(dev_alloc(&m->d_mark_fr, (size_t)m->total));
     A(dev_alloc(&m->d_rows, 4 * (size_t)m->total));
-    A(dev_alloc(&m->d_topen, (size_t)m->total));
-    A(dev_alloc(&m->d_tcost, (size_t)m->total));
     A(dev_alloc(&m->d_ctrl, (size_t)CTL_WORDS));
-    A(dev_alloc(&m->d_cert, 3 * (size_t)nr));
     A(dev_alloc(&m->d_bar, (size_t)BAR_WORDS));
     std::vector<int2> bmap((size_t)m->total);
     for (int r = 0; r < nr; ++r)
@@ -230,10 +228,8 @@ int multi_setup(MultiState* m, Context* const* ctxs, int nr) {
              hipSuccess ||
          hipMemcpy(m->d_bmap, bmap.data(), bmap.size() * sizeof(int2), hipMemcpyHostToDevice) !=
              hipSuccess ||
-         hipMemset(m->d_mark_pf, 0, (size_t)m->total * sizeof(uint32_t)) != hipSuccess ||
          hipMemset(m->d_mark_fr, 0, (size_t)m->total * sizeof(uint32_t)) != hipSuccess ||
          hipMemset(m->d_ctrl, 0, CTL_WORDS * sizeof(uint32_t)) != hipSuccess ||
-         hipMemset(m->d_cert, 0, 3 * (size_t)nr * sizeof(uint32_t)) != hipSuccess ||
          hipMemset(m->d_bar, 0, BAR_WORDS * sizeof(uint32_t)) != hipSuccess))
         st = CAGEO_ERR_HIP;
     // the all-tile launches share the abort word and wait bound of tile 0's
@@ -248,8 +244,8 @@ int multi_setup(MultiState* m, Context* const* ctxs, int nr) {
 }
 
 void multi_release(MultiState* m) {
-    void* ptrs[] = {m->d_base, m->d_bmap, m->d_rinfo, m->d_work, m->d_mark_pf, m->d_mark_fr, m->d_rows, m->d_topen, m->d_tcost, m->d_ctrl,
-                    m->d_cert, m->d_bar, m->d_pf, m->d_fr, m->d_tr};
+    void* ptrs[] = {m->d_base, m->d_bmap, m->d_work, m->d_mark_fr, m->d_rows, m->d_xb, m->d_pfmask, m->d_pfinfo, m->d_ctrl,
+                    m->d_bar, m->d_pf, m->d_fr, m->d_tr};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     *m = MultiState{};

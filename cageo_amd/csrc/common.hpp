@@ -52,10 +52,14 @@ struct Context {
     // tiles
     int ntx = 0, nty = 0, ntiles = 0;
     uint32_t* d_mark = nullptr;  // per-tile epoch stamps of the flat-resolution worklists
-    uint32_t* d_mark_pf = nullptr;  // epoch stamps of the pit-fill kernel
-    uint32_t* d_topen = nullptr;    // per tile: holds OPEN pit-fill cells
-    uint32_t* d_tcost = nullptr;    // per tile: row steps of its last pit-fill solve
     uint32_t* d_rows = nullptr;     // per tile: dirty-row masks, 2 pass parities x 64 bits
+    float* d_xb = nullptr;          // pit fill: 3 x 256 side cells a tile
+    uint2* d_pfmask = nullptr;      // pit fill: cell masks, 256 x 8 bytes a tile
+    uint32_t* d_pfinfo = nullptr;   // pit fill: a word a tile
+    // the pit fill by rounds (pitfill_rounds.hip) only:
+    uint32_t* d_mark_pf = nullptr;  // per tile: epoch stamps
+    uint32_t* d_topen = nullptr;    // per tile: holds OPEN cells
+    uint32_t* d_tcost = nullptr;    // per tile: row steps of its last solve
     int* d_work3 = nullptr;         // 7 worklists of the persistent kernels
     uint32_t* d_ctrl = nullptr;     // control block of the persistent kernels
     uint32_t* d_bar = nullptr;      // grid barrier words (BAR_WORDS), see grid_sync
@@ -355,7 +359,17 @@ enum : int {
     CTL_RESIDENT = 30,  // pit fill: open tiles handed to the resident rounds (0: none)
     CTL_RROUND = 31,    // pit fill: the round the resident rounds go on from
     CTL_FR_DONE = 32,   // flow routing: 1 once the flat passes of the launch converged
-    CTL_WORDS = 33
+    // Pit fill by bounds: four rotating stages of PF_GROUPS lines of 128
+    // bytes, each with a group's tile visits asked for and ended and its
+    // undecided cells at their Z (many workgroups adding to one word queue:
+    // 23 ns each on an MI355X), then the word every workgroup polls.
+    CTL_PF_LINE = 32,
+    CTL_PF_GROUPS = 64,
+    CTL_PF_STAGE = CTL_PF_GROUPS * CTL_PF_LINE,
+    CTL_PF_COUNTS = 64,
+    CTL_PF_OVER = CTL_PF_COUNTS + 4 * CTL_PF_STAGE,  // stages over, or PF_OVER_ABANDON
+    CTL_PF_CLAIM = CTL_PF_OVER + CTL_PF_LINE,        // blocks taken, the first of each workgroup apart
+    CTL_WORDS = CTL_PF_CLAIM + CTL_PF_LINE
 };
 
 // Several rasters in one persistent launch: raster r owns the global 64x64
@@ -379,15 +393,13 @@ struct MultiState {
     int max_cells = 0;                // largest raster (cells)
     int* d_base = nullptr;            // nr + 1 block offsets
     int2* d_bmap = nullptr;           // per block: (raster, block within it)
-    uint2* d_rinfo = nullptr;         // per raster: pit-fill minimum, domain ok
     int* d_work = nullptr;            // 7 lists of `total` entries
-    uint32_t* d_mark_pf = nullptr;    // per-block epoch stamps (pit fill)
+    float* d_xb = nullptr;            // pit fill: 3 x 256 side cells a block
+    uint2* d_pfmask = nullptr;        // pit fill: cell masks, 256 x 8 bytes a block
+    uint32_t* d_pfinfo = nullptr;     // pit fill: a word a block
     uint32_t* d_mark_fr = nullptr;    // per-block epoch stamps (flats)
     uint32_t* d_rows = nullptr;       // per block: dirty-row masks, 2 pass parities x 64 bits
-    uint32_t* d_topen = nullptr;      // per block: holds OPEN pit-fill cells
-    uint32_t* d_tcost = nullptr;      // per block: row steps of its last pit-fill solve
     uint32_t* d_ctrl = nullptr;       // CTL_WORDS
-    uint32_t* d_cert = nullptr;       // 3 rotating counters per raster
     uint32_t* d_bar = nullptr;        // grid barrier words
     const uint32_t* d_habort = nullptr;  // host abort word (the batch's)
     uint64_t bar_limit = 0;
@@ -449,6 +461,9 @@ int realization_body(Context* c, float* mc, hipEvent_t* evs);
 // Its first part: stages a3..a5 and the quantisation into c->d_z.
 int realization_pre(Context* c, hipEvent_t* evs);
 int pit_fill_grid_cap(Context* c, int* cap);
+// The fill by rounds, for callers with a byte a cell of workspace.
+int pit_fill_rounds(Context* c, float* zq, float* w, float nodata);
+int pit_fill_rounds_grid_cap(Context* c, int* cap);
 int pit_fill_resident_cap(Context* c, int* cap);
 int flow_routing_grid_cap(Context* c, int* cap);
 int flow_tracing_grid_cap(Context* c, int* cap);

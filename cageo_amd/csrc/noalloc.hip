@@ -1,9 +1,10 @@
 // Allocation-free pit fill: cageo_pit_fill with its workspace in a file-scope
 // device array instead of a context's allocations, for callers that cannot
 // call hipMalloc (code under HIP graph capture, tight serving loops,
-// harnesses that forbid allocation).  It runs the same kernels as
-// cageo_pit_fill (k_reset_minmax, k_quantize_minmax, k_pf_persistent,
-// k_pf_resident) on the same workspace layout, carved from the array.
+// harnesses that forbid allocation).  Same result as cageo_pit_fill, by the
+// form that needs a byte a cell (pitfill_rounds.hip: k_pf_persistent,
+// k_pf_resident) where cageo_pit_fill's takes 5 KB a tile and a raster of
+// scratch: the array's declared size holds the former only.
 //
 // The array is a __device__ symbol: every device that loads the library holds
 // its own copy, at its own address, until the process ends.  Its host-side
@@ -61,7 +62,7 @@ int device_scratch(int device, DeviceScratch** out) {
         if (!p) return CAGEO_ERR_HIP;
         Context probe;  // host-side settings only: no device memory
         probe.device = device;
-        CAGEO_TRY(pit_fill_grid_cap(&probe, &d.pf_grid));
+        CAGEO_TRY(pit_fill_rounds_grid_cap(&probe, &d.pf_grid));
         CAGEO_TRY(pit_fill_resident_cap(&probe, &d.pf_res_grid));
         CAGEO_TRY(barrier_ticks(device, BAR_DEFAULT_TIMEOUT_S, &d.bar_limit));
         d.ptr = static_cast<uint8_t*>(p);
@@ -135,7 +136,7 @@ extern "C" int cageo_pit_fill_noalloc(float* d_filled, float* d_dem, int width, 
     CAGEO_HIP_TRY(hipGetLastError());
     CAGEO_TRY(reset_minmax(&c));
     CAGEO_TRY(launch_quantize(&c, d_dem, nodata_dem));
-    CAGEO_TRY(pit_fill_quantized(&c, d_dem, d_filled, nodata_dem, true));
+    CAGEO_TRY(pit_fill_rounds(&c, d_dem, d_filled, nodata_dem));
     uint32_t st = 0;
     CAGEO_HIP_TRY(hipMemcpyAsync(&st, c.d_ctrl + CTL_STATUS, sizeof(st), hipMemcpyDeviceToHost,
                                  c.stream));
