@@ -365,82 +365,225 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
 
 // Weight gradient of the 3x3 convolution:
 //   dW[tap][co][ci] += sum_p g[p][co] * x[p shifted by tap][ci]
-// (GEMM rows co, columns ci, K = pixels).  A workgroup takes one tap, a
-// 32x32 (co, ci) block and a run of pixel chunks; each chunk of 32 pixels is
-// staged through LDS (rows of g and of the shifted input are contiguous in
-// NHWC) and read back transposed as MFMA operands.  Partial sums are added
-// to the fp32 gradient with atomics.
-__global__ __launch_bounds__(256) void k_conv3x3_wgrad(ConvIn ci, const uint16_t* __restrict__ g,
-                                                       float* __restrict__ dw, int N, int H, int W,
-                                                       int Cout, int chunks_per_block) {
-    __shared__ uint16_t sg[32][32 + 8];  // [pixel][co]
-    __shared__ uint16_t sx[32][32 + 8];  // [pixel][ci]
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+// (GEMM rows co, columns ci, K = pixels).  A workgroup of 8 waves takes CO
+// output x 32 input channels, all nine taps, over a 64-pixel wide run of image
+// rows, two rows of g a step.
+//
+// Both operands want their channel's pixels in a row (K), but the rasters
+// have a pixel's channels in a row: what is loaded (4 pixels x 8 channels a
+// thread, 16-byte loads) is transposed in registers by byte permutes and
+// stored to LDS channel-major, once for the nine taps.  The row taps are
+// other rows of a ring of six x rows; the column taps are the same 8 pixels
+// shifted by one, made from a fragment and the pixel pairs beside it by five
+// bit alignments.  So a wave's K chunk of 32 pixels takes 2 fragments of g
+// and, per row tap, one of x and two pairs, for 18 MFMAs.
+//
+// A wave owns 32 co x 16 ci x 9 taps (72 accumulator registers).  With CO 64
+// the waves are 2 (co halves) x 2 (ci halves) x 2 (image rows of the step),
+// with CO 32 2 (ci) x 4 (row, pixel half); the partial sums of the waves that
+// share an output are added up in LDS, so a workgroup makes one atomic per
+// weight.  The next step's loads are in flight during a step's MFMAs; one
+// barrier a step.  Strides of 88 (x) and 72 (g) pixels put the 16 channels of
+// a fragment read in distinct bank groups.
+//
+// Bound by the loads' latency at two workgroups a CU.  The kernel it replaced
+// took one tap and 32 x 32 channels a workgroup and read every operand two
+// bytes at a time: 10.8 ms of the 17.3 ms of a step of 8 tiles of 512^2.
+constexpr int WG_T = 512;        // threads
+constexpr int WG_XS = 88;        // pixels of a staged x channel: 8 (pixel -1 last), 64, 1, pad
+constexpr int WG_GS = 72;        // pixels of a staged g channel: 64, pad
+constexpr int WG_XROW = 32 * WG_XS;
+__device__ inline uint32_t pair_lo(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x05040100u); }
+__device__ inline uint32_t pair_hi(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302u); }
+
+template <int CO>
+__global__ __launch_bounds__(WG_T) __attribute__((amdgpu_waves_per_eu(4))) void k_conv3x3_wgrad(
+    ConvIn ci, const uint16_t* __restrict__ g, float* __restrict__ dw, int N, int H, int W, int Cout,
+    int rows) {
+    constexpr int GROW = CO * WG_GS, X_N = 6 * WG_XROW, G_N = 4 * GROW;
+    constexpr int RED_N = 4 * 18 * 256 * 2;  // partial sums of four waves, in bf16 words
+    constexpr int SM_N = X_N + G_N > RED_N ? X_N + G_N : RED_N;
+    __shared__ __align__(16) uint16_t smem[SM_N];
+    uint16_t* const xt = smem;        // [6 ring slots][32 ci][WG_XS]
+    uint16_t* const gt = smem + X_N;  // [2 steps][2 rows][CO][WG_GS]
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int Cin = ci.C1 + ci.C2;
-    const int tap = blockIdx.z % 9;
-    const int dy = tap / 3 - 1, dx = tap % 3 - 1;
-    const int co0 = blockIdx.y * 32;
-    const int ci0 = (blockIdx.z / 9) * 32;
-    const long long M = (long long)N * H * W;
-    // wave (wr, wc) computes the 16x16 block (co0 + 16 wr, ci0 + 16 wc)
-    const int wr = wave >> 1, wc = wave & 1;
-    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-    const long long chunk0 = (long long)blockIdx.x * chunks_per_block;
-    for (int ch = 0; ch < chunks_per_block; ++ch) {
-        const long long pbase = (chunk0 + ch) * 32;
-        if (pbase >= M) break;  // uniform
-        // stage: 256 threads load 32 pixels x 32 channels of g and of x
-        {
-            const int pl = threadIdx.x >> 3, c8 = (threadIdx.x & 7) * 4;  // 4 channels each
-            const long long p = pbase + pl;
-            uint2 gv = make_uint2(0, 0), xv = make_uint2(0, 0);
-            if (p < M) {
-                gv = *reinterpret_cast<const uint2*>(g + p * Cout + co0 + c8);
-                const int n = (int)(p / ((long long)H * W));
-                const int r = (int)(p - (long long)n * H * W);
-                const int y = r / W, x = r - (r / W) * W;
-                const int yy = y + dy, xx = x + dx;
-                if (yy >= 0 && xx >= 0 && yy < H && xx < W) {
-                    const int c = ci0 + c8;
-                    if (c < ci.C1) {
-                        const int H1 = ci.up1 ? (H + 1) / 2 : H, W1 = ci.up1 ? (W + 1) / 2 : W;
-                        const int y1 = ci.up1 ? yy / 2 : yy, x1 = ci.up1 ? xx / 2 : xx;
-                        xv = *reinterpret_cast<const uint2*>(
-                            ci.in1 + (((size_t)n * H1 + y1) * W1 + x1) * ci.C1 + c);
-                    } else {
-                        xv = *reinterpret_cast<const uint2*>(
-                            ci.in2 + (((size_t)n * H + yy) * W + xx) * ci.C2 + (c - ci.C1));
-                    }
+    const int segs = (W + 63) / 64, blocks_y = (H + rows - 1) / rows;
+    const int seg = blockIdx.x % segs, yb = (blockIdx.x / segs) % blocks_y;
+    const int n = blockIdx.x / (segs * blocks_y);
+    const int x0 = seg * 64, y0 = yb * rows, y1 = min(y0 + rows, H);
+    const int co0 = blockIdx.y * CO, ci0 = blockIdx.z * 32;
+
+    // This thread's part of the staging of two rows: 4 pixels x 8 channels of
+    // x (threads 0-127), of g (the next 2 CO x 2), or 8 channels of a pixel
+    // beside the segment (16 more).
+    constexpr int XT = 128, GT = 4 * CO;  // 2 rows x 16 pixel groups x channels / 8
+    static_assert(XT + GT + 16 <= WG_T, "a task a thread");
+    const bool is_x = tid < XT, is_g = tid >= XT && tid < XT + GT;
+    const bool is_h = tid >= XT + GT && tid < XT + GT + 16;
+    int trow, tpx, tc;
+    if (is_g) {
+        const int i = tid - XT;
+        tc = i % (CO / 8);
+        tpx = 4 * ((i / (CO / 8)) & 15);
+        trow = i / (2 * CO);
+    } else if (is_h) {
+        const int i = tid - XT - GT;
+        tc = i & 3;
+        tpx = (i >> 2) & 1 ? 64 : -1;
+        trow = i >> 3;
+    } else {
+        tc = tid & 3;
+        tpx = 4 * ((tid >> 2) & 15);
+        trow = (tid >> 6) & 1;
+    }
+    // the block's 32 input channels lie in one of the two inputs
+    const bool first = ci0 < ci.C1;
+    const uint16_t* const xsrc = first ? ci.in1 : ci.in2;
+    const int xc = first ? ci.C1 : ci.C2, up = first ? ci.up1 : 0;
+    const int xo = (first ? ci0 : ci0 - ci.C1) + 8 * tc;
+    const int Hx = up ? (H + 1) / 2 : H, Wx = up ? (W + 1) / 2 : W;
+    uint4 v[4];
+    // rows y (x: row y0 - 1 + 2 s + trow with s counted two rows ahead of g's)
+    auto load = [&](int xrow, int grow) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = make_uint4(0u, 0u, 0u, 0u);
+        if (is_g) {
+            const int y = grow + trow;
+            if (y >= y1) return;
+            const uint16_t* p = g + (((size_t)n * H + y) * W + x0 + tpx) * Cout + co0 + 8 * tc;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (x0 + tpx + j < W) v[j] = *reinterpret_cast<const uint4*>(p + (size_t)j * Cout);
+        } else if (is_x || is_h) {
+            const int y = xrow + trow;
+            if (y < 0 || y >= H) return;
+            const uint16_t* p = xsrc + ((size_t)n * Hx + (up ? y / 2 : y)) * Wx * xc + xo;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int x = x0 + tpx + j;
+                if (x >= 0 && x < W && (is_x || j == 0))
+                    v[j] = *reinterpret_cast<const uint4*>(p + (size_t)(up ? x / 2 : x) * xc);
+            }
+        }
+    };
+    // slot: ring slot of the first of the two x rows; buf: g's step parity
+    auto store = [&](int slot, int buf) {
+        if (is_h) {
+            const int s = slot + trow;
+            uint16_t* d = xt + (s >= 6 ? s - 6 : s) * WG_XROW + 8 * tc * WG_XS + 8 + tpx;
+            const uint32_t u[4] = {v[0].x, v[0].y, v[0].z, v[0].w};
+#pragma unroll
+            for (int e = 0; e < 8; ++e) d[e * WG_XS] = (uint16_t)(u[e >> 1] >> (16 * (e & 1)));
+            return;
+        }
+        if (!is_x && !is_g) return;
+        const int s = slot + trow;
+        uint16_t* d = is_x ? xt + (s >= 6 ? s - 6 : s) * WG_XROW + 8 * tc * WG_XS + 8 + tpx
+                           : gt + (2 * buf + trow) * GROW + 8 * tc * WG_GS + tpx;
+        const int stride = is_x ? WG_XS : WG_GS;
+        const uint32_t u[4][4] = {{v[0].x, v[0].y, v[0].z, v[0].w}, {v[1].x, v[1].y, v[1].z, v[1].w},
+                                  {v[2].x, v[2].y, v[2].z, v[2].w}, {v[3].x, v[3].y, v[3].z, v[3].w}};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            *reinterpret_cast<uint2*>(d + 2 * k * stride) =
+                make_uint2(pair_lo(u[0][k], u[1][k]), pair_lo(u[2][k], u[3][k]));
+            *reinterpret_cast<uint2*>(d + (2 * k + 1) * stride) =
+                make_uint2(pair_hi(u[0][k], u[1][k]), pair_hi(u[2][k], u[3][k]));
+        }
+    };
+
+    // this wave's share: ci half, then co half and row (CO 64) or row and
+    // pixel half (CO 32)
+    const int wci = wave & 1, wrow = CO == 64 ? wave >> 2 : (wave >> 1) & 1;
+    const int wco = CO == 64 ? (wave >> 1) & 1 : 0;
+    const int c_lo = CO == 64 ? 0 : wave >> 2, c_hi = CO == 64 ? 2 : c_lo + 1;
+    const int row = lane & 15, kb = lane >> 4;
+    f32x4 acc[9][2];
+#pragma unroll
+    for (int t = 0; t < 9; ++t)
+#pragma unroll
+        for (int q = 0; q < 2; ++q) acc[t][q] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    // x rows y0 - 1 .. y0 + 2 and g rows y0, y0 + 1 to begin with
+    load(y0 - 1, y1);
+    store(0, 0);
+    load(y0 + 1, y0);
+    store(2, 0);
+    __syncthreads();
+    int slot = 0;  // ring slot of x row y - 1
+    for (int y = y0, buf = 0; y < y1; y += 2, buf ^= 1) {
+        const bool more = y + 2 < y1;
+        if (more) load(y + 3, y + 2);
+        const uint16_t* gr = gt + (2 * buf + wrow) * GROW + (32 * wco + row) * WG_GS + 8 * kb;
+        for (int c = c_lo; c < c_hi; ++c) {
+            bf16x8 a[2];
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+                a[q] = as_bf16x8(*reinterpret_cast<const uint4*>(gr + 16 * q * WG_GS + 32 * c));
+#pragma unroll
+            for (int dy = 0; dy < 3; ++dy) {
+                int sl = slot + wrow + dy;
+                if (sl >= 6) sl -= 6;
+                const uint16_t* xr = xt + sl * WG_XROW + (16 * wci + row) * WG_XS + 8 + 32 * c + 8 * kb;
+                const uint4 m = *reinterpret_cast<const uint4*>(xr);
+                const uint32_t pv = *reinterpret_cast<const uint32_t*>(xr - 2);
+                const uint32_t nx = *reinterpret_cast<const uint32_t*>(xr + 8);
+                const uint32_t s0 = __builtin_amdgcn_alignbit(m.x, pv, 16);
+                const uint32_t s1 = __builtin_amdgcn_alignbit(m.y, m.x, 16);
+                const uint32_t s2 = __builtin_amdgcn_alignbit(m.z, m.y, 16);
+                const uint32_t s3 = __builtin_amdgcn_alignbit(m.w, m.z, 16);
+                const uint32_t s4 = __builtin_amdgcn_alignbit(nx, m.w, 16);
+                const bf16x8 b0 = as_bf16x8(make_uint4(s0, s1, s2, s3));  // pixel - 1
+                const bf16x8 b1 = as_bf16x8(m);
+                const bf16x8 b2 = as_bf16x8(make_uint4(s1, s2, s3, s4));  // pixel + 1
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    acc[3 * dy][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[q], b0, acc[3 * dy][q], 0, 0, 0);
+                    acc[3 * dy + 1][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[q], b1, acc[3 * dy + 1][q], 0, 0, 0);
+                    acc[3 * dy + 2][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[q], b2, acc[3 * dy + 2][q], 0, 0, 0);
                 }
             }
-            *reinterpret_cast<uint2*>(&sg[pl][c8]) = gv;
-            *reinterpret_cast<uint2*>(&sx[pl][c8]) = xv;
+        }
+        // rows no wave reads in this step: x ring slots 4 and 5 on, the other
+        // g buffer (both last read before the barrier that began the step)
+        if (more) store(slot + 4 >= 6 ? slot - 2 : slot + 4, buf ^ 1);
+        __syncthreads();
+        slot = slot + 2 >= 6 ? slot - 4 : slot + 2;
+    }
+
+    // partial sums of the waves with the same output: CO 64 waves 4-7 into
+    // 0-3; CO 32 waves 4-7 into 0-3, then 2, 3 into 0, 1
+    f32x4* const red = reinterpret_cast<f32x4*>(smem);
+#pragma unroll
+    for (int half = 4; half >= (CO == 64 ? 4 : 2); half >>= 1) {
+        if (wave >= half && wave < 2 * half) {
+#pragma unroll
+            for (int t = 0; t < 9; ++t)
+#pragma unroll
+                for (int q = 0; q < 2; ++q) red[((wave - half) * 18 + 2 * t + q) * 64 + lane] = acc[t][q];
         }
         __syncthreads();
-        // A[i = co][k = pixel], B[k = pixel][j = ci]; lane: row/col l % 16,
-        // pixels 8*(l / 16) .. +7
-        const int i = lane & 15, kb = lane >> 4;
-        uint16_t av[8], bv[8];
+        if (wave < half) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            av[e] = sg[8 * kb + e][16 * wr + i];
-            bv[e] = sx[8 * kb + e][16 * wc + i];
+            for (int t = 0; t < 9; ++t)
+#pragma unroll
+                for (int q = 0; q < 2; ++q) acc[t][q] += red[(wave * 18 + 2 * t + q) * 64 + lane];
         }
-        uint4 a4, b4;
-        a4.x = av[0] | ((uint32_t)av[1] << 16); a4.y = av[2] | ((uint32_t)av[3] << 16);
-        a4.z = av[4] | ((uint32_t)av[5] << 16); a4.w = av[6] | ((uint32_t)av[7] << 16);
-        b4.x = bv[0] | ((uint32_t)bv[1] << 16); b4.y = bv[2] | ((uint32_t)bv[3] << 16);
-        b4.z = bv[4] | ((uint32_t)bv[5] << 16); b4.w = bv[6] | ((uint32_t)bv[7] << 16);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a4), as_bf16x8(b4), acc, 0, 0, 0);
         __syncthreads();
     }
-    const int j = lane & 15, kb = lane >> 4;
+    if (wave >= (CO == 64 ? 4 : 2)) return;
+    // accumulator row 4 kb + r = output channel, column = input channel
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int co = co0 + 16 * wr + 4 * kb + r;
-        const int cix = ci0 + 16 * wc + j;
-        atomicAdd(&dw[((size_t)tap * Cout + co) * Cin + cix], acc[r]);
-    }
+    for (int t = 0; t < 9; ++t)
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                atomicAdd(&dw[((size_t)t * Cout + co0 + 32 * wco + 16 * q + 4 * kb + r) * Cin + ci0 +
+                              16 * wci + row],
+                          acc[t][q][r]);
 }
 
 // ---- elementwise / small kernels ------------------------------------------
@@ -787,19 +930,24 @@ int cageo_nn_conv3x3_wgrad(void* stream, const uint16_t* in1, int c1, int up1,
                            const uint16_t* in2, int c2, const uint16_t* g, float* dw, int n, int h,
                            int wdt, int cout) {
     if (!in1 || !g || !dw || c1 <= 0 || c1 % 32 || c2 % 32 || cout % 32) return CAGEO_ERR_ARG;
+    if (n <= 0 || h <= 0 || wdt <= 0) return CAGEO_OK;  // an empty sum
     ConvIn ci{in1, in2, c1, c2, up1};
-    const long long M = (long long)n * h * wdt;
-    const long long chunks = (M + 31) / 32;
-    const int cin = c1 + c2;
-    // enough workgroups to fill the chip, each over a run of pixel chunks
-    const long long blocks_xy = (long long)(cout / 32) * 9 * (cin / 32);
-    long long bx = (2048 + blocks_xy - 1) / blocks_xy;
-    if (bx > chunks) bx = chunks;
-    if (bx < 1) bx = 1;
-    const int per = (int)((chunks + bx - 1) / bx);
-    dim3 grid((unsigned)((chunks + per - 1) / per), (unsigned)(cout / 32), (unsigned)(9 * (cin / 32)));
-    hipLaunchKernelGGL(k_conv3x3_wgrad, grid, dim3(256), 0, reinterpret_cast<hipStream_t>(stream),
-                       ci, g, dw, n, h, wdt, cout, per);
+    // image rows a workgroup: some 512 workgroups (two a CU), the fewest
+    // atomics that fill the chip; at least 4, the ring's extra rows cost 2
+    const int co = cout % 64 == 0 ? 64 : 32;
+    const long long segs = (wdt + 63) / 64;
+    const long long work = segs * n * h * (cout / co) * ((c1 + c2) / 32);
+    long long rows = std::min<long long>(std::max<long long>((work + 511) / 512, 4), h);
+    rows = (rows + 1) & ~1LL;
+    const dim3 grid((unsigned)(segs * n * ((h + rows - 1) / rows)), (unsigned)(cout / co),
+                    (unsigned)((c1 + c2) / 32));
+    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    if (co == 64)
+        hipLaunchKernelGGL(k_conv3x3_wgrad<64>, grid, dim3(WG_T), 0, st, ci, g, dw, n, h, wdt, cout,
+                           (int)rows);
+    else
+        hipLaunchKernelGGL(k_conv3x3_wgrad<32>, grid, dim3(WG_T), 0, st, ci, g, dw, n, h, wdt, cout,
+                           (int)rows);
     CAGEO_HIP_TRY(hipGetLastError());
     return CAGEO_OK;
 }
