@@ -474,6 +474,10 @@ int flow_tracing(Context* c, const int8_t* fd, const uint8_t* sflags, const int3
                  int32_t* lab, int64_t* long_paths);
 int launch_border(Context* c, float* mc, const int32_t* lab);
 int launch_to_bytes(Context* c, uint8_t* out, const float* in);
+bool nn_conv3x3_fused(void* stream, const uint16_t* in1, int c1, int up1, const uint16_t* in2,
+                      int c2, const uint16_t* w, const float* bias, uint16_t* out, uint16_t* pool,
+                      const float* head_w, const float* head_b, float* prob, int head_sigmoid,
+                      int n, int h, int wdt, int cout, int relu, int* status);
 // Multi-raster launches over the contexts of a batch (tables built once by
 // multi_setup; each context's working buffers are used as in the one-raster
 // stages: pit fill d_z -> d_w, routing d_w -> d_fd, tracing d_fd -> d_lab).

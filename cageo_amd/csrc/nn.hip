@@ -131,8 +131,9 @@ __global__ __launch_bounds__(256) void k_conv3x3(ConvIn ci, const uint16_t* __re
     }
 }
 
-// The same convolution with its operands staged in LDS, for W % 64 == 0 and
-// H % (4 RW) == 0.  A workgroup computes a tile of 4 RW rows x 64 pixels
+// The same convolution with its operands staged in LDS, for any W and H (the
+// tiles at the right and lower edges load zeros and store what lies inside).
+// A workgroup computes a tile of 4 RW rows x 64 pixels
 // (wave w: rows w RW .. w RW + RW - 1, 4 accumulator tiles of 16 pixels
 // each) x 16*NT output channels; with RW = 2 each weight fragment read
 // feeds twice the MFMAs (the 32-channel layers).  Per 32-channel slice of
@@ -167,7 +168,9 @@ struct ConvFuse {
     int sigmoid;
 };
 
-template <int NT, int RW, int WPE>
+// EDGE: W or H is no multiple of the tile's (else the stores need no tests:
+// with them a 4096^2 prediction takes 2 % longer).
+template <int NT, int RW, int WPE, bool EDGE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void k_conv3x3_lds(ConvIn ci, const uint16_t* __restrict__ w,
                                                      const float* __restrict__ bias,
                                                      uint16_t* __restrict__ out,
@@ -185,7 +188,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
     uint16_t* const sb = smem + SA_N;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int row = lane & 15, kb = lane >> 4;
-    const int tiles_x = W / CL_TX, tiles_y = H / TY;
+    const int tiles_x = EDGE ? (W + CL_TX - 1) / CL_TX : W / CL_TX;
+    const int tiles_y = EDGE ? (H + TY - 1) / TY : H / TY;
     const int t = blockIdx.x;
     const int n = t / (tiles_x * tiles_y);
     const int ty = (t / tiles_x) % tiles_y, tx = t % tiles_x;
@@ -275,6 +279,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
     }
     if (outf) {  // fp32 output too: straight from the accumulators
         const long long prow = ((long long)n * H + y0 + wave * RW) * W + x0;
+        const int wy = H - y0 - wave * RW, wx = W - x0;  // the tile's rows and pixels inside
 #pragma unroll
         for (int q = 0; q < NT; ++q) {
             const int co = co0 + 16 * q + row;  // accumulator column = lane % 16
@@ -283,6 +288,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
             for (int m = 0; m < 4 * RW; ++m)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
+                    if (EDGE && (m / 4 >= wy || 16 * (m % 4) + 4 * kb + r >= wx)) continue;
                     const long long pp = prow + (long long)(m / 4) * W + 16 * (m % 4) + 4 * kb + r;
                     float v = acc[m][q][r] + bias_co;
                     if (relu) v = fmaxf(v, 0.0f);
@@ -315,6 +321,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
     __syncthreads();
     if (head) {  // CO == Cout (the host checks): the workgroup holds every channel
         for (int px = threadIdx.x; px < NPX; px += 256) {
+            if (EDGE && (px / CL_TX >= H - y0 || px % CL_TX >= W - x0)) continue;
             float s = fz.head_b[0];
             for (int c = 0; c < CO; ++c) s += fz.head_w[c] * bf2f(smem[c * HP + px]);
             fz.prob[pix0 + (size_t)(px / CL_TX) * W + px % CL_TX] =
@@ -326,6 +333,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
     if (out) {
         for (int i = threadIdx.x; i < NPX * CH; i += 256) {
             const int px = i / CH, part = i - px * CH;
+            if (EDGE && (px / CL_TX >= H - y0 || px % CL_TX >= W - x0)) continue;
             const size_t g = (pix0 + (size_t)(px / CL_TX) * W + px % CL_TX) * Cout + co0 + 8 * part;
             *reinterpret_cast<uint4*>(out + g) =
                 *reinterpret_cast<const uint4*>(smem + px * PS + 8 * part);
@@ -337,6 +345,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
         for (int i = threadIdx.x; i < NPX / 4 * CH; i += 256) {
             const int pp = i / CH, part = i - pp * CH;
             const int py = pp / (CL_TX / 2), px = pp - py * (CL_TX / 2);
+            if (EDGE && (2 * py >= H - y0 || 2 * px >= W - x0)) continue;
             const uint16_t* s00 = smem + (2 * py * CL_TX + 2 * px) * PS + 8 * part;
             const uint4 a = *reinterpret_cast<const uint4*>(s00);                 // (2y, 2x)
             const uint4 b = *reinterpret_cast<const uint4*>(s00 + PS);            // (2y, 2x+1)
@@ -842,10 +851,16 @@ int grid_for(long long n) {
 
 }  // namespace
 
-// The LDS-staged convolution applies: whole 64-pixel row segments, whole
-// 4-row blocks, output channels in blocks of 32.
-inline bool lds_conv_applies(int h, int wdt, int cout) {
-    return wdt % CL_TX == 0 && h % 4 == 0 && cout % 32 == 0;
+// The LDS-staged convolution is the faster one where output channels come in
+// blocks of 32, unless most of a large launch would be padding: with at least
+// a quarter of its 4 x 64 tiles' pixels in the image (2000 x 24 x 64 -> 64
+// channels: 15 us against 33), or at most two workgroups a CU (8 x 16 x 16:
+// 11 against 32).  On narrower ones the other kernel, whose waves take pixels
+// of several rows, does less.
+inline bool lds_conv_applies(int n, int h, int wdt, int cout) {
+    const long long tiles = (long long)n * ((h + 3) / 4) * ((wdt + CL_TX - 1) / CL_TX);
+    return cout % 32 == 0 && (4LL * n * h * wdt >= tiles * 4 * CL_TX ||
+                              tiles * (cout % 64 == 0 ? cout / 64 : cout / 32) <= 512);
 }
 // Output channels of one workgroup of the LDS-staged convolution.
 inline int lds_conv_block(int cout) { return cout % 64 == 0 ? 64 : 32; }
@@ -860,15 +875,37 @@ int launch_conv_lds(void* stream, const ConvIn& ci, const uint16_t* w, const flo
                     uint16_t* out, float* outf, const ConvFuse& fz, int n, int h, int wdt, int cout,
                     int relu) {
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    const unsigned tx = (unsigned)(wdt / CL_TX);
-    if (cout % 64 == 0)
-        hipLaunchKernelGGL((k_conv3x3_lds<4, 1, 2>), dim3((unsigned)n * (h / 4) * tx, cout / 64),
-                           dim3(256), 0, st, ci, w, bias, out, outf, fz, n, h, wdt, cout, relu);
-    else
-        hipLaunchKernelGGL((k_conv3x3_lds<2, 1, 3>), dim3((unsigned)n * (h / 4) * tx, cout / 32),
-                           dim3(256), 0, st, ci, w, bias, out, outf, fz, n, h, wdt, cout, relu);
+    const unsigned tiles = (unsigned)n * ((h + 3) / 4) * ((wdt + CL_TX - 1) / CL_TX);
+    auto launch = [&](auto kernel, int block) {
+        hipLaunchKernelGGL(kernel, dim3(tiles, cout / block), dim3(256), 0, st, ci, w, bias, out,
+                           outf, fz, n, h, wdt, cout, relu);
+    };
+    const bool edge = wdt % CL_TX != 0 || h % 4 != 0;
+    if (cout % 64 == 0) {
+        if (edge) launch(k_conv3x3_lds<4, 1, 2, true>, 64);
+        else launch(k_conv3x3_lds<4, 1, 2, false>, 64);
+    } else {
+        if (edge) launch(k_conv3x3_lds<2, 1, 3, true>, 32);
+        else launch(k_conv3x3_lds<2, 1, 3, false>, 32);
+    }
     CAGEO_HIP_TRY(hipGetLastError());
     return CAGEO_OK;
+}
+
+// The forward convolution with fused consumers wherever the staged kernel
+// takes the image (the C ABI's fused call promises whole tiles only): returns
+// false, with nothing launched, where it does not.
+bool nn_conv3x3_fused(void* stream, const uint16_t* in1, int c1, int up1, const uint16_t* in2,
+                      int c2, const uint16_t* w, const float* bias, uint16_t* out, uint16_t* pool,
+                      const float* head_w, const float* head_b, float* prob, int head_sigmoid,
+                      int n, int h, int wdt, int cout, int relu, int* status) {
+    if (!lds_conv_applies(n, h, wdt, cout) || (pool && (h % 2 || wdt % 2)) ||
+        (prob && lds_conv_block(cout) != cout))
+        return false;
+    const ConvIn ci{in1, in2, c1, c2, up1};
+    const ConvFuse fz{pool, head_w, head_b, prob, head_sigmoid};
+    *status = launch_conv_lds(stream, ci, w, bias, out, nullptr, fz, n, h, wdt, cout, relu);
+    return true;
 }
 
 }  // namespace cageo
@@ -885,7 +922,7 @@ int cageo_nn_conv3x3(void* stream, const uint16_t* in1, int c1, int up1, const u
     if (c1 <= 0 || c1 % 32 || c2 < 0 || c2 % 32 || (c2 && !in2) || cout % 16) return CAGEO_ERR_ARG;
     ConvIn ci{in1, in2, c1, c2, up1};
     const long long M = (long long)n * h * wdt;
-    if (lds_conv_applies(h, wdt, cout))
+    if (lds_conv_applies(n, h, wdt, cout))
         return launch_conv_lds(stream, ci, w, bias, out, outf, ConvFuse{}, n, h, wdt, cout, relu);
     // output channel tile: 64 (NT 4), 32 (NT 2) or 16 (NT 1); 4 pixel tiles
     // per wave (256 pixels per workgroup; 8 lowered occupancy and time)
@@ -907,7 +944,7 @@ int cageo_nn_conv3x3(void* stream, const uint16_t* in1, int c1, int up1, const u
 }
 
 int cageo_nn_conv3x3_fusable(int h, int wdt, int cout, int head) {
-    if (h <= 0 || wdt <= 0 || cout <= 0 || !lds_conv_applies(h, wdt, cout)) return 0;
+    if (h <= 0 || wdt <= 0 || cout <= 0 || wdt % CL_TX || h % 4 || cout % 32) return 0;
     return head ? (lds_conv_block(cout) == cout ? 1 : 0) : 1;
 }
 

@@ -27,11 +27,6 @@ int cageo_nn_conv3x3(void* stream, const uint16_t* in1, int c1, int up1, const u
 int cageo_nn_avgpool2(void* stream, const uint16_t* in, uint16_t* out, int n, int h, int w, int c);
 int cageo_nn_head(void* stream, const uint16_t* act, const float* w, const float* b, float* logit,
                   long long p, int c, int sigmoid);
-int cageo_nn_conv3x3_fusable(int h, int w, int cout, int head);
-int cageo_nn_conv3x3_fused(void* stream, const uint16_t* in1, int c1, int up1, const uint16_t* in2,
-                           int c2, const uint16_t* w, const float* bias, uint16_t* out,
-                           uint16_t* pool, const float* head_w, const float* head_b, float* prob,
-                           int head_sigmoid, int n, int h, int wdt, int cout, int relu);
 }
 
 namespace cageo {
@@ -334,11 +329,11 @@ int conv_pool(cageo_surrogate* s, const char* name, const uint16_t* in1, int c1,
     auto wi = s->dev.find(n + ".w"), bi = s->dev.find(n + ".b");
     if (wi == s->dev.end() || bi == s->dev.end()) return CAGEO_ERR_STATE;
     const int cout = s->shape[n + ".b"][0];
-    if (cageo_nn_conv3x3_fusable(h, w, cout, 0))
-        return cageo_nn_conv3x3_fused(s->stream, in1, c1, 0, nullptr, 0,
-                                      static_cast<const uint16_t*>(wi->second),
-                                      static_cast<const float*>(bi->second), out, pooled, nullptr,
-                                      nullptr, nullptr, 0, 1, h, w, cout, 1);
+    int st = CAGEO_OK;
+    if (nn_conv3x3_fused(s->stream, in1, c1, 0, nullptr, 0, static_cast<const uint16_t*>(wi->second),
+                         static_cast<const float*>(bi->second), out, pooled, nullptr, nullptr,
+                         nullptr, 0, 1, h, w, cout, 1, &st))
+        return st;
     CAGEO_TRY(conv(s, name, in1, c1, 0, nullptr, 0, out, h, w));
     return cageo_nn_avgpool2(s->stream, out, pooled, 1, h, w, cout);
 }
@@ -355,11 +350,11 @@ int conv_head(cageo_surrogate* s, const char* name, const uint16_t* in1, int c1,
     const int cout = s->shape[n + ".b"][0];
     const float* hw = static_cast<const float*>(s->dev["head.w"]);
     const float* hb = static_cast<const float*>(s->dev["head.b"]);
-    if (cageo_nn_conv3x3_fusable(h, w, cout, 1))
-        return cageo_nn_conv3x3_fused(s->stream, in1, c1, 0, nullptr, 0,
-                                      static_cast<const uint16_t*>(wi->second),
-                                      static_cast<const float*>(bi->second), nullptr, nullptr, hw,
-                                      hb, s->prob_pad, 1, 1, h, w, cout, 1);
+    int st = CAGEO_OK;
+    if (nn_conv3x3_fused(s->stream, in1, c1, 0, nullptr, 0, static_cast<const uint16_t*>(wi->second),
+                         static_cast<const float*>(bi->second), nullptr, nullptr, hw, hb,
+                         s->prob_pad, 1, 1, h, w, cout, 1, &st))
+        return st;
     CAGEO_TRY(conv(s, name, in1, c1, 0, nullptr, 0, tmp, h, w));
     return cageo_nn_head(s->stream, tmp, hw, hb, s->prob_pad, (long long)h * w, cout, 1);
 }
