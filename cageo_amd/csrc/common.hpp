@@ -474,6 +474,21 @@ int flow_tracing(Context* c, const int8_t* fd, const uint8_t* sflags, const int3
                  int32_t* lab, int64_t* long_paths);
 int launch_border(Context* c, float* mc, const int32_t* lab);
 int launch_to_bytes(Context* c, uint8_t* out, const float* in);
+// Partial sums of a bias gradient: slots of workgroups, added up at the end.
+constexpr int BIAS_SLOTS = 64;
+int nn_dgrad_relu(void* stream, const uint16_t* g, int co, const uint16_t* wt, const uint16_t* act,
+                  uint16_t* gout, float* dbias, int n, int h, int w, int cin);
+int nn_head_back_relu(void* stream, const uint16_t* act, const float* w, const float* logit,
+                      const float* target, float* q, uint16_t* gout, float* dw, float* db,
+                      float* loss, float* dbias, long long p, int c);
+int nn_up_relu_back(void* stream, const float* dy, const uint16_t* act, uint16_t* g, float* dbias,
+                    int n, int h, int w, int c, int ctot);
+int nn_skip_relu_back(void* stream, const float* dcat, int ctot, int coff, const float* dp,
+                      const uint16_t* act, uint16_t* g, float* dbias, int n, int h, int w, int c);
+int nn_bias_sums(void* stream, int layers, const float* const* part, float* const* db,
+                 const int* c);
+int nn_flip_all(void* stream, int layers, const uint16_t* const* w, uint16_t* const* wt,
+                const int* cout, const int* cin);
 bool nn_conv3x3_fused(void* stream, const uint16_t* in1, int c1, int up1, const uint16_t* in2,
                       int c2, const uint16_t* w, const float* bias, uint16_t* out, uint16_t* pool,
                       const float* head_w, const float* head_b, float* prob, int head_sigmoid,

@@ -166,7 +166,52 @@ struct ConvFuse {
     const float* head_b;
     float* prob;          // [N][H][W] head output, or null (then head_w/head_b unused)
     int sigmoid;
+    // a data gradient's ReLU backward: the output is masked by mask > 0
+    // (bf16 [N][H][W][Cout]), and its sums over the pixels, the bias gradient
+    // of the layer that made `mask`, go to dbias ([BIAS_SLOTS][Cout] partials)
+    const uint16_t* mask;
+    float* dbias;
 };
+
+// 0xffff halves where the bf16 halves of `a` are positive (a ReLU's output is
+// never NaN).
+__device__ inline uint32_t positive_halves(uint32_t a) {
+    const uint32_t lo = (a & 0x8000u) == 0u && (a & 0x7fffu) != 0u ? 0xffffu : 0u;
+    const uint32_t hi = (a & 0x80000000u) == 0u && (a & 0x7fff0000u) != 0u ? 0xffff0000u : 0u;
+    return lo | hi;
+}
+__device__ inline uint4 relu_mask(uint4 v, uint4 a) {
+    return make_uint4(v.x & positive_halves(a.x), v.y & positive_halves(a.y),
+                      v.z & positive_halves(a.z), v.w & positive_halves(a.w));
+}
+// Adds 8 bf16 values to 8 sums.
+__device__ inline void add8(float (&s)[8], uint4 v) {
+    const uint32_t u[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        s[2 * k] += bf2f((uint16_t)(u[k] & 0xffffu));
+        s[2 * k + 1] += bf2f((uint16_t)(u[k] >> 16));
+    }
+}
+// Sums over the workgroup (256 threads) of each thread's 8 channels
+// 8 (threadIdx.x % CH) .. + 7, CH a power of two up to 32, added to this
+// workgroup's slot of the partial sums: atomics of thousands of workgroups on
+// one row of words would queue (23 ns each).  `part`: 4 x 8 CH floats of LDS.
+__device__ inline void bias_partials(float (&s)[8], int CH, float* part, float* dbias, int cout,
+                                     int co0) {
+    for (int off = 32; off >= CH; off >>= 1)
+#pragma unroll
+        for (int k = 0; k < 8; ++k) s[k] += __shfl_xor(s[k], off);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, C = 8 * CH;
+    if (lane < CH)
+#pragma unroll
+        for (int k = 0; k < 8; ++k) part[wave * C + 8 * lane + k] = s[k];
+    __syncthreads();
+    if ((int)threadIdx.x < C)
+        atomicAdd(&dbias[(size_t)(blockIdx.x % BIAS_SLOTS) * cout + co0 + threadIdx.x],
+                  (part[threadIdx.x] + part[C + threadIdx.x]) +
+                      (part[2 * C + threadIdx.x] + part[3 * C + threadIdx.x]));
+}
 
 // EDGE: W or H is no multiple of the tile's (else the stores need no tests:
 // with them a 4096^2 prediction takes 2 % longer).
@@ -330,6 +375,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
         return;
     }
     constexpr int CH = CO / 8;  // 16-byte chunks of a pixel's channels
+    if (fz.mask) {
+        float sum[8] = {};
+#pragma unroll
+        for (int i0 = 0; i0 < NPX * CH; i0 += 256) {
+            const int i = i0 + threadIdx.x, px = i / CH, part = i - px * CH;
+            if (EDGE && (px / CL_TX >= H - y0 || px % CL_TX >= W - x0)) continue;
+            const size_t o = (pix0 + (size_t)(px / CL_TX) * W + px % CL_TX) * Cout + co0 + 8 * part;
+            const uint4 v = relu_mask(*reinterpret_cast<const uint4*>(smem + px * PS + 8 * part),
+                                      *reinterpret_cast<const uint4*>(fz.mask + o));
+            *reinterpret_cast<uint4*>(out + o) = v;
+            add8(sum, v);
+        }
+        __syncthreads();  // the staged outputs are read
+        bias_partials(sum, CH, reinterpret_cast<float*>(smem), fz.dbias, Cout, co0);
+        return;
+    }
     if (out) {
         for (int i = threadIdx.x; i < NPX * CH; i += 256) {
             const int px = i / CH, part = i - px * CH;
@@ -701,6 +762,120 @@ __global__ __launch_bounds__(256) void k_relu_back_bias(const float* __restrict_
     }
 }
 
+// Gradient of an upsampled tensor through its upsampling and the ReLU that
+// made it (act): g = bf16(act > 0 ? sum of dy's 2x2 block : 0), dy the first C
+// of Ctot channels at twice the size, and the sums of g as dbias partials.
+// One pass where k_upsample2_back and k_relu_back_bias took two, and the
+// tensor in between was stored: 0.27 ms of a 512^2 x 8 step's level 1 before,
+// 0.15 now.  A thread takes 8 channels; 8 * 256 is a multiple of C.
+__global__ __launch_bounds__(256) void k_up_relu_back(const float* __restrict__ dy,
+                                                      const uint16_t* __restrict__ act,
+                                                      uint16_t* __restrict__ g, int N, int H, int W,
+                                                      int C, int Ctot, float* __restrict__ dbias) {
+    __shared__ float part[4 * 256];
+    const int Ho = H / 2, Wo = W / 2, CH = C / 8;
+    float sum[8] = {};
+    GRID_STRIDE(i, (long long)N * Ho * Wo * CH) {
+        const long long p = i / CH;
+        const int c = 8 * (int)(i - p * CH);
+        const int x = (int)(p % Wo);
+        const long long ny = p / Wo;
+        const int y = (int)(ny % Ho);
+        const size_t n = (size_t)(ny / Ho);
+        const float* d = dy + ((n * H + 2 * y) * W + 2 * x) * Ctot + c;
+        const size_t off[4] = {0, (size_t)Ctot, (size_t)W * Ctot, (size_t)W * Ctot + Ctot};
+        float4 v[4][2];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            v[k][0] = *reinterpret_cast<const float4*>(d + off[k]);
+            v[k][1] = *reinterpret_cast<const float4*>(d + off[k] + 4);
+        }
+        const uint4 a = *reinterpret_cast<const uint4*>(act + p * C + c);
+        uint32_t m[4];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const float4 &q0 = v[0][h], &q1 = v[1][h], &q2 = v[2][h], &q3 = v[3][h];
+            m[2 * h] = (uint32_t)f2bf(((q0.x + q1.x) + q2.x) + q3.x) |
+                       ((uint32_t)f2bf(((q0.y + q1.y) + q2.y) + q3.y) << 16);
+            m[2 * h + 1] = (uint32_t)f2bf(((q0.z + q1.z) + q2.z) + q3.z) |
+                           ((uint32_t)f2bf(((q0.w + q1.w) + q2.w) + q3.w) << 16);
+        }
+        const uint4 r = relu_mask(make_uint4(m[0], m[1], m[2], m[3]), a);
+        *reinterpret_cast<uint4*>(g + p * C + c) = r;
+        add8(sum, r);
+    }
+    bias_partials(sum, CH, part, dbias, C, 0);
+}
+
+// Gradient of an encoder output through the ReLU that made it: the decoder's
+// share (channels coff.. of dcat's Ctot) plus a quarter of the pooled
+// tensor's, g = bf16(act > 0 ? dcat + dp / 4 : 0), and dbias partials.  In
+// place of k_slice_add, k_avgpool2_back and k_relu_back_bias.
+__global__ __launch_bounds__(256) void k_skip_relu_back(const float* __restrict__ dcat, int Ctot,
+                                                        int coff, const float* __restrict__ dp,
+                                                        const uint16_t* __restrict__ act,
+                                                        uint16_t* __restrict__ g, int N, int H,
+                                                        int W, int C, float* __restrict__ dbias) {
+    __shared__ float part[4 * 256];
+    const int CH = C / 8;
+    float sum[8] = {};
+    GRID_STRIDE(i, (long long)N * H * W * CH) {
+        const long long p = i / CH;
+        const int c = 8 * (int)(i - p * CH);
+        const int x = (int)(p % W);
+        const long long ny = p / W;
+        const int y = (int)(ny % H);
+        const size_t n = (size_t)(ny / H);
+        const float4* s = reinterpret_cast<const float4*>(dcat + (size_t)p * Ctot + coff + c);
+        const float4* q = reinterpret_cast<const float4*>(
+            dp + ((n * (H / 2) + y / 2) * (W / 2) + x / 2) * C + c);
+        const float4 s0 = s[0], s1 = s[1], q0 = q[0], q1 = q[1];
+        const uint4 a = *reinterpret_cast<const uint4*>(act + p * C + c);
+        const uint4 v = make_uint4(
+            (uint32_t)f2bf(s0.x + 0.25f * q0.x) | ((uint32_t)f2bf(s0.y + 0.25f * q0.y) << 16),
+            (uint32_t)f2bf(s0.z + 0.25f * q0.z) | ((uint32_t)f2bf(s0.w + 0.25f * q0.w) << 16),
+            (uint32_t)f2bf(s1.x + 0.25f * q1.x) | ((uint32_t)f2bf(s1.y + 0.25f * q1.y) << 16),
+            (uint32_t)f2bf(s1.z + 0.25f * q1.z) | ((uint32_t)f2bf(s1.w + 0.25f * q1.w) << 16));
+        const uint4 r = relu_mask(v, a);
+        *reinterpret_cast<uint4*>(g + p * C + c) = r;
+        add8(sum, r);
+    }
+    bias_partials(sum, CH, part, dbias, C, 0);
+}
+
+// Bias gradients of every layer from their partials.
+struct BiasTable {
+    static constexpr int MAX = 16;
+    const float* part[MAX];
+    float* db[MAX];
+    int c[MAX];
+};
+__global__ void k_bias_sum(BiasTable t) {
+    const int l = blockIdx.x, c = threadIdx.x;
+    if (c >= t.c[l]) return;
+    float s = 0.0f;
+#pragma unroll 16
+    for (int k = 0; k < BIAS_SLOTS; ++k) s += t.part[l][(size_t)k * t.c[l] + c];
+    t.db[l][c] += s;
+}
+
+// Weights of the data-gradient convolutions of every layer (k_flip_transpose).
+struct FlipTable {
+    static constexpr int MAX = 16;
+    const uint16_t* w[MAX];
+    uint16_t* wt[MAX];
+    int cout[MAX], cin[MAX];
+};
+__global__ void k_flip_all(FlipTable t) {
+    const int l = blockIdx.y, Cout = t.cout[l], Cin = t.cin[l];
+    GRID_STRIDE(i, 9LL * Cout * Cin) {
+        // output order: consecutive threads write consecutive words
+        const int co = (int)(i % Cout);
+        const int r = (int)(i / Cout), ci = r % Cin, tap = r / Cin;
+        t.wt[l][i] = t.w[l][((size_t)(8 - tap) * Cout + co) * Cin + ci];
+    }
+}
+
 // Bias gradient: db[c] += sum_p g[p][c] (g bf16).
 __global__ void k_bias_grad(const uint16_t* __restrict__ g, float* __restrict__ db, long long P,
                             int C) {
@@ -744,23 +919,35 @@ __global__ void k_head(const uint16_t* __restrict__ act, const float* __restrict
 // multiple of 32 up to HEAD_MAX_C: each thread sums its pixels' terms of
 // the weight gradient in registers, a workgroup adds them up in LDS and
 // makes one atomic per channel.
+// MASK: d(act) goes out behind the ReLU that made act, rounded to bf16 (gout),
+// with its sums over the pixels in dbias (BIAS_SLOTS partials), instead of
+// fp32 into dact.
 constexpr int HEAD_MAX_C = 128;
-template <int C>
+template <int C, bool MASK>
 __global__ __launch_bounds__(256) void k_head_back(const uint16_t* __restrict__ act,
                                                    const float* __restrict__ w,
                                                    const float* __restrict__ logit,
                                                    const float* __restrict__ target,
                                                    float* __restrict__ q, float* __restrict__ dact,
                                                    float* __restrict__ dw, float* __restrict__ db,
-                                                   float* __restrict__ loss, long long P) {
+                                                   float* __restrict__ loss, long long P,
+                                                   uint16_t* __restrict__ gout,
+                                                   float* __restrict__ dbias) {
     __shared__ float part[C];
+    __shared__ float bpart[MASK ? C : 1];
     __shared__ float red[2];
-    for (int c = threadIdx.x; c < C; c += blockDim.x) part[c] = 0.0f;
+    for (int c = threadIdx.x; c < C; c += blockDim.x) {
+        part[c] = 0.0f;
+        if (MASK) bpart[c] = 0.0f;
+    }
     if (threadIdx.x < 2) red[threadIdx.x] = 0.0f;
     __syncthreads();
-    float acc[C];
+    float acc[C], bacc[MASK ? C : 1];
 #pragma unroll
-    for (int c = 0; c < C; ++c) acc[c] = 0.0f;
+    for (int c = 0; c < C; ++c) {
+        acc[c] = 0.0f;
+        if (MASK) bacc[c] = 0.0f;
+    }
     float lsum = 0.0f, bsum = 0.0f;
     GRID_STRIDE(p, P) {
         const float z = logit[p];
@@ -777,11 +964,22 @@ __global__ __launch_bounds__(256) void k_head_back(const uint16_t* __restrict__ 
         for (int c8 = 0; c8 < C / 8; ++c8) {
             const uint4 v = a[c8];
             const uint32_t u[4] = {v.x, v.y, v.z, v.w};
+            uint32_t m[4];
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 const int c = 8 * c8 + 2 * k;
                 acc[c] += g * bf2f((uint16_t)(u[k] & 0xffffu));
                 acc[c + 1] += g * bf2f((uint16_t)(u[k] >> 16));
+                if (MASK) {
+                    m[k] = ((uint32_t)f2bf(g * w[c]) | ((uint32_t)f2bf(g * w[c + 1]) << 16)) &
+                           positive_halves(u[k]);
+                    bacc[c] += bf2f((uint16_t)(m[k] & 0xffffu));
+                    bacc[c + 1] += bf2f((uint16_t)(m[k] >> 16));
+                }
+            }
+            if (MASK) {
+                reinterpret_cast<uint4*>(gout + p * C)[c8] = make_uint4(m[0], m[1], m[2], m[3]);
+                continue;
             }
             d[2 * c8] = make_float4(g * w[8 * c8], g * w[8 * c8 + 1], g * w[8 * c8 + 2], g * w[8 * c8 + 3]);
             d[2 * c8 + 1] = make_float4(g * w[8 * c8 + 4], g * w[8 * c8 + 5], g * w[8 * c8 + 6],
@@ -793,6 +991,11 @@ __global__ __launch_bounds__(256) void k_head_back(const uint16_t* __restrict__ 
         float v = acc[c];
         for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
         if ((threadIdx.x & 63) == 0) atomicAdd(&part[c], v);
+        if (MASK) {
+            float bv = bacc[c];
+            for (int off = 32; off > 0; off >>= 1) bv += __shfl_xor(bv, off);
+            if ((threadIdx.x & 63) == 0) atomicAdd(&bpart[c], bv);
+        }
     }
     for (int off = 32; off > 0; off >>= 1) {
         lsum += __shfl_xor(lsum, off);
@@ -803,7 +1006,10 @@ __global__ __launch_bounds__(256) void k_head_back(const uint16_t* __restrict__ 
         atomicAdd(&red[1], bsum);
     }
     __syncthreads();
-    for (int c = threadIdx.x; c < C; c += blockDim.x) atomicAdd(&dw[c], part[c]);
+    for (int c = threadIdx.x; c < C; c += blockDim.x) {
+        atomicAdd(&dw[c], part[c]);
+        if (MASK) atomicAdd(&dbias[(size_t)(blockIdx.x % BIAS_SLOTS) * C + c], bpart[c]);
+    }
     if (threadIdx.x == 0) {
         atomicAdd(loss, red[0] / (float)P);
         atomicAdd(db, red[1]);
@@ -888,6 +1094,76 @@ int launch_conv_lds(void* stream, const ConvIn& ci, const uint16_t* w, const flo
         if (edge) launch(k_conv3x3_lds<2, 1, 3, true>, 32);
         else launch(k_conv3x3_lds<2, 1, 3, false>, 32);
     }
+    CAGEO_HIP_TRY(hipGetLastError());
+    return CAGEO_OK;
+}
+
+// The backward passes of the trainer: see the kernels.  Channel counts are
+// powers of two of at most 256 (the trainer checks); `n` images of h x w.
+int nn_dgrad_relu(void* stream, const uint16_t* g, int co, const uint16_t* wt, const uint16_t* act,
+                  uint16_t* gout, float* dbias, int n, int h, int w, int cin) {
+    const ConvIn ci{g, nullptr, co, 0, 0};
+    ConvFuse fz{};
+    fz.mask = act;
+    fz.dbias = dbias;
+    return launch_conv_lds(stream, ci, wt, nullptr, gout, nullptr, fz, n, h, w, cin, 0);
+}
+int nn_head_back_relu(void* stream, const uint16_t* act, const float* w, const float* logit,
+                      const float* target, float* q, uint16_t* gout, float* dw, float* db,
+                      float* loss, float* dbias, long long p, int c) {
+    if (c != 32) return CAGEO_ERR_ARG;
+    const int grid = (int)std::min<long long>(1024, (p + 255) / 256);
+    hipLaunchKernelGGL((k_head_back<32, true>), dim3(grid), dim3(256), 0,
+                       reinterpret_cast<hipStream_t>(stream), act, w, logit, target, q,
+                       (float*)nullptr, dw, db, loss, p, gout, dbias);
+    CAGEO_HIP_TRY(hipGetLastError());
+    return CAGEO_OK;
+}
+int nn_up_relu_back(void* stream, const float* dy, const uint16_t* act, uint16_t* g, float* dbias,
+                    int n, int h, int w, int c, int ctot) {
+    const long long work = (long long)n * (h / 2) * (w / 2) * (c / 8);
+    const int grid = (int)std::min<long long>(2048, (work + 255) / 256);
+    hipLaunchKernelGGL(k_up_relu_back, dim3(grid), dim3(256), 0,
+                       reinterpret_cast<hipStream_t>(stream), dy, act, g, n, h, w, c, ctot, dbias);
+    CAGEO_HIP_TRY(hipGetLastError());
+    return CAGEO_OK;
+}
+int nn_skip_relu_back(void* stream, const float* dcat, int ctot, int coff, const float* dp,
+                      const uint16_t* act, uint16_t* g, float* dbias, int n, int h, int w, int c) {
+    const long long work = (long long)n * h * w * (c / 8);
+    const int grid = (int)std::min<long long>(2048, (work + 255) / 256);
+    hipLaunchKernelGGL(k_skip_relu_back, dim3(grid), dim3(256), 0,
+                       reinterpret_cast<hipStream_t>(stream), dcat, ctot, coff, dp, act, g, n, h, w,
+                       c, dbias);
+    CAGEO_HIP_TRY(hipGetLastError());
+    return CAGEO_OK;
+}
+int nn_bias_sums(void* stream, int layers, const float* const* part, float* const* db,
+                 const int* c) {
+    if (layers > BiasTable::MAX) return CAGEO_ERR_ARG;
+    BiasTable t{};
+    for (int l = 0; l < layers; ++l) {
+        t.part[l] = part[l];
+        t.db[l] = db[l];
+        t.c[l] = c[l];
+    }
+    hipLaunchKernelGGL(k_bias_sum, dim3(layers), dim3(256), 0,
+                       reinterpret_cast<hipStream_t>(stream), t);
+    CAGEO_HIP_TRY(hipGetLastError());
+    return CAGEO_OK;
+}
+int nn_flip_all(void* stream, int layers, const uint16_t* const* w, uint16_t* const* wt,
+                const int* cout, const int* cin) {
+    if (layers > FlipTable::MAX) return CAGEO_ERR_ARG;
+    FlipTable t{};
+    for (int l = 0; l < layers; ++l) {
+        t.w[l] = w[l];
+        t.wt[l] = wt[l];
+        t.cout[l] = cout[l];
+        t.cin[l] = cin[l];
+    }
+    hipLaunchKernelGGL(k_flip_all, dim3(128, layers), dim3(256), 0,
+                       reinterpret_cast<hipStream_t>(stream), t);
     CAGEO_HIP_TRY(hipGetLastError());
     return CAGEO_OK;
 }
@@ -1060,17 +1336,21 @@ int cageo_nn_head_back(void* stream, const uint16_t* act, const float* w, const 
     const int grid = (int)std::min<long long>(1024, (p + 255) / 256);
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     if (c == 32)
-        hipLaunchKernelGGL(k_head_back<32>, dim3(grid), dim3(256), 0, s, act, w, logit, target, q,
-                           dact, dw, db, loss, p);
+        hipLaunchKernelGGL((k_head_back<32, false>), dim3(grid), dim3(256), 0, s, act, w, logit, target, q,
+                           dact, dw, db, loss, p, (uint16_t*)nullptr,
+                           (float*)nullptr);
     else if (c == 64)
-        hipLaunchKernelGGL(k_head_back<64>, dim3(grid), dim3(256), 0, s, act, w, logit, target, q,
-                           dact, dw, db, loss, p);
+        hipLaunchKernelGGL((k_head_back<64, false>), dim3(grid), dim3(256), 0, s, act, w, logit, target, q,
+                           dact, dw, db, loss, p, (uint16_t*)nullptr,
+                           (float*)nullptr);
     else if (c == 96)
-        hipLaunchKernelGGL(k_head_back<96>, dim3(grid), dim3(256), 0, s, act, w, logit, target, q,
-                           dact, dw, db, loss, p);
+        hipLaunchKernelGGL((k_head_back<96, false>), dim3(grid), dim3(256), 0, s, act, w, logit, target, q,
+                           dact, dw, db, loss, p, (uint16_t*)nullptr,
+                           (float*)nullptr);
     else if (c == HEAD_MAX_C)
-        hipLaunchKernelGGL(k_head_back<HEAD_MAX_C>, dim3(grid), dim3(256), 0, s, act, w, logit,
-                           target, q, dact, dw, db, loss, p);
+        hipLaunchKernelGGL((k_head_back<HEAD_MAX_C, false>), dim3(grid), dim3(256), 0, s, act, w, logit,
+                           target, q, dact, dw, db, loss, p, (uint16_t*)nullptr,
+                           (float*)nullptr);
     else
         return CAGEO_ERR_ARG;
     CAGEO_HIP_TRY(hipGetLastError());

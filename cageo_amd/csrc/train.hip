@@ -37,6 +37,7 @@ constexpr TrLayer TR_LAYERS[] = {
     {"mida", 4, 0, 0, 8, 3},  {"midb", 8, 0, 0, 8, 3},  {"dec3a", 8, 1, 4, 4, 2},
     {"dec3b", 4, 0, 0, 4, 2}, {"dec2a", 4, 1, 2, 2, 1}, {"dec2b", 2, 0, 0, 2, 1},
     {"dec1a", 2, 1, 1, 1, 0}, {"dec1b", 1, 0, 0, 1, 0}};
+enum { E1A, E1B, E2A, E2B, E3A, E3B, MA, MB, D3A, D3B, D2A, D2B, D1A, D1B };
 constexpr int TR_NLAYERS = sizeof(TR_LAYERS) / sizeof(TR_LAYERS[0]);
 
 struct Param {
@@ -132,8 +133,11 @@ struct cageo_trainer {
     std::vector<uint16_t*> act;  // forward activations, see forward()
     float *logit = nullptr, *q = nullptr;
     std::vector<float*> gr;      // backward gradients, see backward()
-    uint16_t* gtmp = nullptr;    // bf16 output gradient of the layer being differentiated
-    uint16_t* wt = nullptr;      // flipped, transposed weights of that layer
+    uint16_t* gb[2] = {};        // bf16 output gradients of the layer being differentiated, the next
+    std::vector<uint16_t*> wt;   // flipped, transposed weights (layers from the second on)
+    float* slab = nullptr;       // every parameter's gradient, then the bias partials
+    long long slab_n = 0;
+    std::vector<float*> bpart;   // per layer: BIAS_SLOTS x channels
     float* loss = nullptr;       // per-step losses of the running loop
     int loss_cap = 0;
     int* sel = nullptr;          // batch selections of the running loop
@@ -158,7 +162,7 @@ void free_batch(cageo_trainer* t) {
     t->xb = nullptr;
     t->yb = nullptr;
     t->logit = t->q = nullptr;
-    t->gtmp = t->wt = nullptr;
+    t->gb[0] = t->gb[1] = nullptr;
     t->n = t->h = t->w = 0;
 }
 
@@ -195,36 +199,27 @@ int ensure_batch(cageo_trainer* t, int n, int h, int w) {
     }
     CAGEO_TRY(alloc(t, &t->logit, P));
     CAGEO_TRY(alloc(t, &t->q, P));
-    // backward: per layer the gradient of its output (fp32) and, for the
-    // decoder's first layers, of its concatenated input
-    for (const TrLayer& L : TR_LAYERS) {
+    // backward: fp32 gradients of the decoder's concatenated inputs (levels
+    // 0-2) and of the pooled tensors (levels 1-3)
+    for (int i : {D1A, D2A, D3A}) {
         float* g = nullptr;
-        CAGEO_TRY(alloc(t, &g, px(L.level) * L.com * b));
+        const TrLayer& L = TR_LAYERS[i];
+        CAGEO_TRY(alloc(t, &g, px(L.level) * (L.c1m + L.c2m) * b));
         t->gr.push_back(g);
     }
-    for (const TrLayer& L : TR_LAYERS) {
-        float* g = nullptr;
-        const int cin = L.c1m == 0 ? TR_IN_PAD : (L.c1m + L.c2m) * b;
-        CAGEO_TRY(alloc(t, &g, L.up1 ? px(L.level) * cin : 1));
-        t->gr.push_back(g);
-    }
-    for (int lv = 1; lv <= 3; ++lv) {  // gradients of the pooled tensors
+    for (int lv = 1; lv <= 3; ++lv) {
         float* g = nullptr;
         CAGEO_TRY(alloc(t, &g, px(lv) * (b << (lv - 1))));
         t->gr.push_back(g);
     }
-    CAGEO_TRY(alloc(t, &t->gtmp, P * b));  // the largest layer output: b channels at full size
-    size_t wmax = 0;  // the largest 9 x cin x cout
-    for (const TrLayer& L : TR_LAYERS)
-        wmax = std::max(wmax, (size_t)9 * (L.c1m == 0 ? TR_IN_PAD : (L.c1m + L.c2m) * b) * L.com * b);
-    CAGEO_TRY(alloc(t, &t->wt, wmax));
+    // the largest layer output: b channels at full size
+    CAGEO_TRY(alloc(t, &t->gb[0], P * b));
+    CAGEO_TRY(alloc(t, &t->gb[1], P * b));
     t->n = n;
     t->h = h;
     t->w = w;
     return CAGEO_OK;
 }
-
-enum { E1A, E1B, E2A, E2B, E3A, E3B, MA, MB, D3A, D3B, D2A, D2B, D1A, D1B };
 
 // Inputs of layer i: in1 (c1 channels; upsampled with up1) and in2 (c2).
 struct LayerIn {
@@ -263,12 +258,19 @@ int forward(cageo_trainer* t) {
         const LayerIn in = layer_in(t, i);
         Param* w = find(t, std::string(L.name) + ".w");
         Param* bias = find(t, std::string(L.name) + ".b");
-        CAGEO_TRY(cageo_nn_conv3x3(s, in.in1, in.c1, in.up1, in.in2, in.c2, w->pb, bias->p,
-                                   t->act[i], nullptr, n, t->h >> L.level, t->w >> L.level,
-                                   L.com * b, 1));
+        const int lv = L.level;
         // the encoder outputs of levels 0-2 are pooled for the next level
-        if (i == E1B || i == E2B || i == E3B) {
-            const int lv = L.level;
+        const bool pool = i == E1B || i == E2B || i == E3B;
+        int st = CAGEO_OK;
+        if (pool && nn_conv3x3_fused(s, in.in1, in.c1, in.up1, in.in2, in.c2, w->pb, bias->p,
+                                     t->act[i], t->act[TR_NLAYERS + lv], nullptr, nullptr, nullptr,
+                                     0, n, t->h >> lv, t->w >> lv, L.com * b, 1, &st)) {
+            CAGEO_TRY(st);
+            continue;
+        }
+        CAGEO_TRY(cageo_nn_conv3x3(s, in.in1, in.c1, in.up1, in.in2, in.c2, w->pb, bias->p,
+                                   t->act[i], nullptr, n, t->h >> lv, t->w >> lv, L.com * b, 1));
+        if (pool) {
             CAGEO_TRY(cageo_nn_avgpool2(s, t->act[i], t->act[TR_NLAYERS + lv], n, t->h >> lv,
                                         t->w >> lv, L.com * b));
         }
@@ -277,31 +279,30 @@ int forward(cageo_trainer* t) {
                          (long long)n * t->h * t->w, b, 0);
 }
 
-// Gradients of layer i from the fp32 gradient of its output: bias and
-// weight gradients (added), and with need_dx the gradient of its input
-// (fp32, its concatenated channels) into dx.
-int layer_back(cageo_trainer* t, int i, const float* gout, float* dx) {
-    const TrLayer& L = TR_LAYERS[i];
-    const int b = t->base, n = t->n, h = t->h >> L.level, w = t->w >> L.level;
-    const int co = L.com * b;
-    const long long P = (long long)n * h * w;
-    void* s = t->stream;
-    const LayerIn in = layer_in(t, i);
-    Param* pw = find(t, std::string(L.name) + ".w");
-    Param* pb = find(t, std::string(L.name) + ".b");
-    CAGEO_TRY(cageo_nn_relu_back_bias(s, gout, t->act[i], t->gtmp, P, co, pb->g));
-    CAGEO_TRY(cageo_nn_conv3x3_wgrad(s, in.in1, in.c1, in.up1, in.in2, in.c2, t->gtmp, pw->g, n,
-                                     h, w, co));
-    if (!dx) return CAGEO_OK;
-    const int cin = in.c1 + in.c2;
-    CAGEO_TRY(cageo_nn_flip_transpose(s, pw->pb, t->wt, co, cin));
-    return cageo_nn_conv3x3(s, t->gtmp, co, 0, nullptr, 0, t->wt, nullptr, nullptr, dx, n, h, w,
-                            cin, 0);
-}
-
 int zero(cageo_trainer* t, float* p, long long n) {
     hipLaunchKernelGGL(k_tr_zero, dim3(tr_grid(n)), dim3(256), 0, t->stream, p, n);
     CAGEO_HIP_TRY(hipGetLastError());
+    return CAGEO_OK;
+}
+
+// Weight gradient of layer i from the bf16 gradient of its output, and the
+// gradient of its input: behind the ReLU of layer `prev`, whose output that
+// input is, as bf16 into gout (with the sums for prev's bias gradient), or in
+// fp32 into dx; neither for the first layer.
+int layer_back(cageo_trainer* t, int i, const uint16_t* g, int prev, uint16_t* gout, float* dx) {
+    const TrLayer& L = TR_LAYERS[i];
+    const int b = t->base, n = t->n, h = t->h >> L.level, w = t->w >> L.level;
+    const int co = L.com * b;
+    void* s = t->stream;
+    const LayerIn in = layer_in(t, i);
+    CAGEO_TRY(cageo_nn_conv3x3_wgrad(s, in.in1, in.c1, in.up1, in.in2, in.c2, g,
+                                     t->params[2 * i].g, n, h, w, co));
+    const int cin = in.c1 + in.c2;
+    if (gout)
+        return nn_dgrad_relu(s, g, co, t->wt[i], t->act[prev], gout, t->bpart[prev], n, h, w, cin);
+    if (dx)
+        return cageo_nn_conv3x3(s, g, co, 0, nullptr, 0, t->wt[i], nullptr, nullptr, dx, n, h, w,
+                                cin, 0);
     return CAGEO_OK;
 }
 
@@ -309,47 +310,58 @@ int zero(cageo_trainer* t, float* p, long long n) {
 // batch's mean BCE added to *d_loss.
 int backward(cageo_trainer* t, float* d_loss) {
     const int b = t->base, n = t->n, h = t->h, w = t->w;
+    // the bias sums take power-of-two channel counts up to 256
+    if (b != 32) return CAGEO_ERR_ARG;
     void* s = t->stream;
-    auto px = [&](int lv) { return (long long)n * (h >> lv) * (w >> lv); };
-    float* const* G = t->gr.data();        // G[i]: gradient of layer i's output
-    float* const* DC = t->gr.data() + TR_NLAYERS;  // DC[i]: of its concatenated input (up1 layers)
-    float* const* DP = t->gr.data() + 2 * TR_NLAYERS;  // DP[lv-1]: of pooled tensor lv
-    for (Param& p : t->params) CAGEO_TRY(zero(t, p.g, p.n));
+    const auto& A = t->act;
+    float* const* DC = t->gr.data();      // of the concatenated inputs of D1A, D2A, D3A
+    float* const* DP = t->gr.data() + 3;  // DP[lv-1]: of pooled tensor lv
+    uint16_t *ga = t->gb[0], *gb = t->gb[1];
+    CAGEO_TRY(zero(t, t->slab, t->slab_n));
+    {
+        const uint16_t* wsrc[TR_NLAYERS];
+        int co[TR_NLAYERS], cin[TR_NLAYERS];
+        for (int i = 1; i < TR_NLAYERS; ++i) {
+            wsrc[i - 1] = t->params[2 * i].pb;
+            co[i - 1] = TR_LAYERS[i].com * b;
+            cin[i - 1] = (TR_LAYERS[i].c1m + TR_LAYERS[i].c2m) * b;
+        }
+        CAGEO_TRY(nn_flip_all(s, TR_NLAYERS - 1, wsrc, t->wt.data() + 1, co, cin));
+    }
     Param* hw = find(t, "head.w");
     Param* hb = find(t, "head.b");
-    CAGEO_TRY(cageo_nn_head_back(s, t->act[D1B], hw->p, t->logit, t->yb, t->q, G[D1B], hw->g,
-                                 hb->g, d_loss, px(0), b));
-    // decoder level 1 (full resolution)
-    CAGEO_TRY(layer_back(t, D1B, G[D1B], G[D1A]));
-    CAGEO_TRY(layer_back(t, D1A, G[D1A], DC[D1A]));                       // [2b up | b]
-    CAGEO_TRY(cageo_nn_slice_add(s, DC[D1A], G[E1B], px(0), b, 3 * b, 2 * b, 0));
-    CAGEO_TRY(zero(t, G[D2B], px(1) * 2 * b));
-    CAGEO_TRY(cageo_nn_upsample2_back(s, DC[D1A], G[D2B], n, h, w, 2 * b, 3 * b, 0));
-    // level 2
-    CAGEO_TRY(layer_back(t, D2B, G[D2B], G[D2A]));
-    CAGEO_TRY(layer_back(t, D2A, G[D2A], DC[D2A]));                       // [4b up | 2b]
-    CAGEO_TRY(cageo_nn_slice_add(s, DC[D2A], G[E2B], px(1), 2 * b, 6 * b, 4 * b, 0));
-    CAGEO_TRY(zero(t, G[D3B], px(2) * 4 * b));
-    CAGEO_TRY(cageo_nn_upsample2_back(s, DC[D2A], G[D3B], n, h >> 1, w >> 1, 4 * b, 6 * b, 0));
-    // level 3
-    CAGEO_TRY(layer_back(t, D3B, G[D3B], G[D3A]));
-    CAGEO_TRY(layer_back(t, D3A, G[D3A], DC[D3A]));                       // [8b up | 4b]
-    CAGEO_TRY(cageo_nn_slice_add(s, DC[D3A], G[E3B], px(2), 4 * b, 12 * b, 8 * b, 0));
-    CAGEO_TRY(zero(t, G[MB], px(3) * 8 * b));
-    CAGEO_TRY(cageo_nn_upsample2_back(s, DC[D3A], G[MB], n, h >> 2, w >> 2, 8 * b, 12 * b, 0));
-    // middle
-    CAGEO_TRY(layer_back(t, MB, G[MB], G[MA]));
-    CAGEO_TRY(layer_back(t, MA, G[MA], DP[2]));
-    CAGEO_TRY(cageo_nn_avgpool2_back(s, DP[2], G[E3B], n, h >> 2, w >> 2, 4 * b));
-    // encoder
-    CAGEO_TRY(layer_back(t, E3B, G[E3B], G[E3A]));
-    CAGEO_TRY(layer_back(t, E3A, G[E3A], DP[1]));
-    CAGEO_TRY(cageo_nn_avgpool2_back(s, DP[1], G[E2B], n, h >> 1, w >> 1, 2 * b));
-    CAGEO_TRY(layer_back(t, E2B, G[E2B], G[E2A]));
-    CAGEO_TRY(layer_back(t, E2A, G[E2A], DP[0]));
-    CAGEO_TRY(cageo_nn_avgpool2_back(s, DP[0], G[E1B], n, h, w, b));
-    CAGEO_TRY(layer_back(t, E1B, G[E1B], G[E1A]));
-    CAGEO_TRY(layer_back(t, E1A, G[E1A], nullptr));
+    CAGEO_TRY(nn_head_back_relu(s, A[D1B], hw->p, t->logit, t->yb, t->q, ga, hw->g, hb->g, d_loss,
+                                t->bpart[D1B], (long long)n * h * w, b));
+    // decoder: level 0 (full resolution) first.  A level's second layer, then
+    // its first, whose input is [the coarser level upsampled | the skip]
+    constexpr int SECOND[3] = {D1B, D2B, D3B}, FIRST[3] = {D1A, D2A, D3A}, BELOW[3] = {D2B, D3B, MB};
+    for (int lv = 0; lv < 3; ++lv) {
+        CAGEO_TRY(layer_back(t, SECOND[lv], ga, FIRST[lv], gb, nullptr));
+        CAGEO_TRY(layer_back(t, FIRST[lv], gb, -1, nullptr, DC[lv]));
+        const int c = 2 * b << lv;  // channels of the coarser level
+        CAGEO_TRY(nn_up_relu_back(s, DC[lv], A[BELOW[lv]], ga, t->bpart[BELOW[lv]], n, h >> lv,
+                                  w >> lv, c, c + c / 2));
+    }
+    CAGEO_TRY(layer_back(t, MB, ga, MA, gb, nullptr));
+    CAGEO_TRY(layer_back(t, MA, gb, -1, nullptr, DP[2]));
+    // encoder: a level's output went to the decoder and, pooled, to the level below
+    constexpr int ESECOND[3] = {E1B, E2B, E3B}, EFIRST[3] = {E1A, E2A, E3A};
+    for (int lv = 2; lv >= 0; --lv) {
+        const int c = b << lv;
+        CAGEO_TRY(nn_skip_relu_back(s, DC[lv], 3 * c, 2 * c, DP[lv], A[ESECOND[lv]], ga,
+                                    t->bpart[ESECOND[lv]], n, h >> lv, w >> lv, c));
+        CAGEO_TRY(layer_back(t, ESECOND[lv], ga, EFIRST[lv], gb, nullptr));
+        CAGEO_TRY(layer_back(t, EFIRST[lv], gb, -1, nullptr, lv > 0 ? DP[lv - 1] : nullptr));
+    }
+    {
+        float* db[TR_NLAYERS];
+        int c[TR_NLAYERS];
+        for (int i = 0; i < TR_NLAYERS; ++i) {
+            db[i] = t->params[2 * i + 1].g;
+            c[i] = TR_LAYERS[i].com * b;
+        }
+        CAGEO_TRY(nn_bias_sums(s, TR_NLAYERS, t->bpart.data(), db, c));
+    }
     Param* w1 = find(t, "enc1a.w");
     hipLaunchKernelGGL(k_tr_zero_pad, dim3(tr_grid(9LL * b * (TR_IN_PAD - TR_IN_CH))), dim3(256),
                        0, t->stream, w1->g, 9LL * b, TR_IN_PAD, TR_IN_CH);
@@ -417,17 +429,36 @@ int make_params(cageo_trainer* t) {
         for (int d : p.shape) p.n *= d;
         const size_t bytes = (size_t)p.n * sizeof(float);
         if (hipMalloc(reinterpret_cast<void**>(&p.p), bytes) != hipSuccess ||
-            hipMalloc(reinterpret_cast<void**>(&p.g), bytes) != hipSuccess ||
             hipMalloc(reinterpret_cast<void**>(&p.m), bytes) != hipSuccess ||
             hipMalloc(reinterpret_cast<void**>(&p.v), bytes) != hipSuccess)
             return CAGEO_ERR_NOMEM;
         CAGEO_HIP_TRY(hipMemset(p.m, 0, bytes));
         CAGEO_HIP_TRY(hipMemset(p.v, 0, bytes));
-        CAGEO_HIP_TRY(hipMemset(p.g, 0, bytes));
         if (p.shape.size() == 3 &&
             hipMalloc(reinterpret_cast<void**>(&p.pb), (size_t)p.n * sizeof(uint16_t)) != hipSuccess)
             return CAGEO_ERR_NOMEM;
     }
+    // the gradients and the bias partials in one piece: cleared at once
+    auto up = [](long long n) { return (n + 63) & ~63LL; };
+    for (const Param& p : t->params) t->slab_n += up(p.n);
+    for (const TrLayer& L : TR_LAYERS) t->slab_n += (long long)BIAS_SLOTS * L.com * b;
+    if (hipMalloc(reinterpret_cast<void**>(&t->slab), (size_t)t->slab_n * sizeof(float)) != hipSuccess)
+        return CAGEO_ERR_NOMEM;
+    CAGEO_HIP_TRY(hipMemset(t->slab, 0, (size_t)t->slab_n * sizeof(float)));
+    float* q = t->slab;
+    for (Param& p : t->params) {
+        p.g = q;
+        q += up(p.n);
+    }
+    for (const TrLayer& L : TR_LAYERS) {
+        t->bpart.push_back(q);
+        q += (long long)BIAS_SLOTS * L.com * b;
+    }
+    t->wt.assign(TR_NLAYERS, nullptr);
+    for (int i = 1; i < TR_NLAYERS; ++i)
+        if (hipMalloc(reinterpret_cast<void**>(&t->wt[i]),
+                      (size_t)t->params[2 * i].n * sizeof(uint16_t)) != hipSuccess)
+            return CAGEO_ERR_NOMEM;
     return CAGEO_OK;
 }
 
@@ -531,10 +562,13 @@ int cageo_trainer_destroy(cageo_trainer* t) {
     else (void)hipDeviceSynchronize();
     cageo::free_batch(t);
     for (Param& p : t->params) {
-        for (float* q : {p.p, p.g, p.m, p.v})
+        for (float* q : {p.p, p.m, p.v})
             if (q) (void)hipFree(q);
         if (p.pb) (void)hipFree(p.pb);
     }
+    for (uint16_t* q : t->wt)
+        if (q) (void)hipFree(q);
+    if (t->slab) (void)hipFree(t->slab);
     if (t->loss) (void)hipFree(t->loss);
     if (t->sel) (void)hipFree(t->sel);
     delete t;
