@@ -52,9 +52,9 @@ struct Context {
     // tiles
     int ntx = 0, nty = 0, ntiles = 0;
     uint32_t* d_mark = nullptr;  // per-tile epoch stamps of the flat-resolution worklists
-    uint32_t* d_rows = nullptr;     // per tile: dirty-row masks, 2 pass parities x 64 bits
+    uint32_t* d_rows = nullptr;     // pit fill, per tile: dirty-row masks, 2 parities x 64 bits
     float* d_xb = nullptr;          // pit fill: 3 x 256 side cells a tile
-    uint2* d_pfmask = nullptr;      // pit fill: cell masks, 256 x 8 bytes a tile
+    uint2* d_pfmask = nullptr;      // cell masks, 256 x 8 bytes a tile: of the pit fill, then of the flats
     uint32_t* d_pfinfo = nullptr;   // pit fill: a word a tile
     // the pit fill by rounds (pitfill_rounds.hip) only:
     uint32_t* d_mark_pf = nullptr;  // per tile: epoch stamps
@@ -117,7 +117,7 @@ struct Context {
     int32_t* d_dist = nullptr;
     int32_t* d_lab = nullptr;
     uint64_t* d_ptr = nullptr;
-    uint64_t* d_bent = nullptr;  // flow tracing: 256 border-table slots per tile
+    uint64_t* d_bent = nullptr;  // 256 words per tile: the flats' masks, then the tracing's border table
 
     // timing
     bool timing = false;
@@ -395,10 +395,10 @@ struct MultiState {
     int2* d_bmap = nullptr;           // per block: (raster, block within it)
     int* d_work = nullptr;            // 7 lists of `total` entries
     float* d_xb = nullptr;            // pit fill: 3 x 256 side cells a block
-    uint2* d_pfmask = nullptr;        // pit fill: cell masks, 256 x 8 bytes a block
+    uint2* d_pfmask = nullptr;        // as the context's, a block
     uint32_t* d_pfinfo = nullptr;     // pit fill: a word a block
     uint32_t* d_mark_fr = nullptr;    // per-block epoch stamps (flats)
-    uint32_t* d_rows = nullptr;       // per block: dirty-row masks, 2 pass parities x 64 bits
+    uint32_t* d_rows = nullptr;       // pit fill, per block: dirty-row masks, 2 parities x 64 bits
     uint32_t* d_ctrl = nullptr;       // CTL_WORDS
     uint32_t* d_bar = nullptr;        // grid barrier words
     const uint32_t* d_habort = nullptr;  // host abort word (the batch's)

@@ -30,6 +30,7 @@
 // raster order) are counted.  performConnectFlowPath (:115-134) then maps a
 // label >= 0 (only 0 occurs: labels are -stream <= 0 or the negative
 // constants) to label[0] when that is negative; it is applied in step 3.
+#include <algorithm>
 #include <vector>
 
 #include "common.hpp"
@@ -429,7 +430,8 @@ int flow_tracing(Context* c, const int8_t* fd, const uint8_t* sflags, const int3
     a.gb = context_gridbar(c);
     hipLaunchKernelGGL(k_tr_tiles<false>, dim3(a.total), dim3(TILE_THREADS), 0, c->stream, a);
     // ordinary launch within the occupancy cap (see pit_fill_quantized)
-    hipLaunchKernelGGL(k_tr_jump<false>, dim3(c->tr_grid), dim3(TILE_THREADS), 0, c->stream, a);
+    hipLaunchKernelGGL(k_tr_jump<false>, dim3(std::min(c->tr_grid, a.total)), dim3(TILE_THREADS), 0,
+                       c->stream, a);
     hipLaunchKernelGGL(k_tr_exits<false>, dim3(a.total), dim3(TILE_THREADS), 0, c->stream, a);
     CAGEO_HIP_TRY(hipGetLastError());
     if (long_paths) {
@@ -465,7 +467,7 @@ int flow_tracing_multi(MultiState* m, hipStream_t s) {
     a.ctrl = m->d_ctrl;
     a.gb = multi_gridbar(m);
     hipLaunchKernelGGL(k_tr_tiles<true>, dim3(a.total), dim3(TILE_THREADS), 0, s, a);
-    hipLaunchKernelGGL(k_tr_jump<true>, dim3(m->tr_grid), dim3(TILE_THREADS), 0, s, a);
+    hipLaunchKernelGGL(k_tr_jump<true>, dim3(std::min(m->tr_grid, a.total)), dim3(TILE_THREADS), 0, s, a);
     hipLaunchKernelGGL(k_tr_exits<true>, dim3(a.total), dim3(TILE_THREADS), 0, s, a);
     CAGEO_HIP_TRY(hipGetLastError());
     return CAGEO_OK;
