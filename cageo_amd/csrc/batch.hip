@@ -203,7 +203,6 @@ int multi_setup(MultiState* m, Context* const* ctxs, int nr) {
     std::vector<int> base(nr + 1, 0);
     for (int r = 0; r < nr; ++r) {
         base[r + 1] = base[r] + ctxs[r]->ntiles;
-        m->max_cells = std::max(m->max_cells, (int)ctxs[r]->n);
     }
     m->total = base[nr];
     int st = CAGEO_OK;

@@ -390,7 +390,6 @@ __device__ inline long long wave_unit_stride() { return (long long)gridDim.x * (
 // per-raster buffers stay in each raster's context).
 struct MultiState {
     int nr = 0, total = 0;            // rasters, global 64x64 blocks
-    int max_cells = 0;                // largest raster (cells)
     int* d_base = nullptr;            // nr + 1 block offsets
     int2* d_bmap = nullptr;           // per block: (raster, block within it)
     int* d_work = nullptr;            // 7 lists of `total` entries
