@@ -63,18 +63,19 @@ def test_one_path(ca, torch_cuda, h, w, down, workgroups):
 
 @pytest.mark.parametrize("side", [2, 63, 64, 65, 150])
 def test_cycles(ca, torch_cuda, side):
-    """A square ring of cells that lead round, every other cell towards it."""
+    """A square ring of cells that lead round, and a row above it into it."""
     announce("cycle", side)
     h, w = 211, 260
-    y0, x0 = 40, 50
+    y0, x0 = 1, 50
     fd = np.zeros((h, w, 2), np.int8)
-    fd[..., 0] = np.where(np.arange(w) < x0, 1, -1)[None]
+    fd[..., 1] = 1  # out of the grid
     y1, x1 = y0 + side - 1, x0 + side - 1
     fd[y0, x0:x1] = (1, 0)
     fd[y0:y1, x1] = (0, 1)
     fd[y1, x0 + 1:x1 + 1] = (-1, 0)
     fd[y0 + 1:y1 + 1, x0] = (0, -1)
     stream = np.full((h, w), NODATA, np.float32)
+    stream[y0 + 1:y1, x0 + 1:x1] = 2.0
     trace(ca, torch_cuda, fd, stream)
-    stream[::37, ::41] = 5.0
+    stream[y1, (x0 + x1) // 2] = 5.0  # opens the ring
     trace(ca, torch_cuda, fd, stream)
