@@ -116,7 +116,7 @@ struct Context {
     int8_t* d_fd = nullptr;
     int32_t* d_dist = nullptr;
     int32_t* d_lab = nullptr;
-    uint64_t* d_ptr = nullptr;
+    uint64_t* d_ptr = nullptr;   // scratch of the checks
     uint64_t* d_bent = nullptr;  // 256 words per tile: the flats' masks, then the tracing's border table
 
     // timing

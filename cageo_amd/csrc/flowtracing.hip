@@ -8,14 +8,15 @@
 // cycle) leaves its path at 0.  A cell's label is therefore the label of its
 // path's terminal, computed here by pointer jumping in two levels:
 //   1. per 64x64 tile, in LDS: every cell's pointer jumps along the in-tile
-//      part of its path (12 doubling rounds cover 4096 cells) and ends as a
-//      terminal label, "stuck" (its path cycles inside the tile, e.g. a cell
-//      without a direction), or an exit: the first cell outside the tile.
-//      Cells that end in their tile get their label at once.  An exit lands
-//      on a border cell of the neighbouring tile, so the tile also writes the
+//      part of its path (12 doubling rounds cover 4096 cells) and ends at a
+//      cell whose label is known, is "stuck" (its path cycles inside the
+//      tile, e.g. a cell without a direction), or ends at a cell that exits
+//      to another tile.  Cells of the first kind get their label at once, the
+//      last keep the exit's slot and their steps to it as a positive code in
+//      the label raster.  An exit lies on the tile's border and lands on a
+//      border cell of the neighbouring tile, so the tile also writes the
 //      entries of its own 252 border cells into a compact border table
-//      (256 slots per tile), and each exit cell keeps the border slot it
-//      exits to and its step count;
+//      (256 slots per tile);
 //   2. over the border table only: exits jump through the entries of the
 //      slots they name, in place, until no exit is left; a chain of more
 //      steps than the raster has cells, or of more hops than there are slots,
@@ -24,8 +25,8 @@
 //      rewritten, names a slot on that cell's own path with the step count to
 //      it, so a hop through either is correct, and a rewritten one is further
 //      along;
-//   3. every exit cell takes the label its border slot resolved to.
-// Entries are 64 bits: kind (2 bits) | steps (30 bits) | value (32 bits), so
+//   3. every exit cell takes the label its tile's border slot resolved to.
+// Table entries are 64 bits: kind (2 bits) | steps (30 bits) | value (32 bits), so
 // the step count to the terminal is known and cells whose terminal is more
 // than 100 001 steps away (where the reference's result depends on its
 // raster order) are counted.  performConnectFlowPath (:115-134) then maps a
@@ -42,20 +43,17 @@ namespace {
 
 constexpr uint32_t K_LOCAL = 0, K_RESOLVED = 1, K_EXIT = 2, K_STUCK = 3;
 constexpr uint64_t STEP_MASK = (1ull << 30) - 1;
-// Label of an exit cell between steps 1 and 3 (labels are -stream ids, at
-// least -2^31 + 1, or the negative constants, or 0).
-constexpr int32_t EXIT_MARK = INT32_MIN;
 constexpr int BORDER_SLOTS = 256;
 
 // Slot of tile cell (lx, ly) in its tile's border table: row 0 -> 0..63,
 // row 63 -> 64..127, column 0 (rows 1..62) -> 129..190, column 63 (rows
 // 1..62) -> 193..254; -1 inside.  Slots 128, 191, 192 and 255 stay unused.
 __device__ inline int border_slot(int lx, int ly) {
-    if (ly == 0) return lx;
-    if (ly == TILE - 1) return TILE + lx;
-    if (lx == 0) return 2 * TILE + ly;
-    if (lx == TILE - 1) return 3 * TILE + ly;
-    return -1;
+    int s = -1;
+    s = lx == TILE - 1 ? 3 * TILE + ly : s;
+    s = lx == 0 ? 2 * TILE + ly : s;
+    s = ly == TILE - 1 ? TILE + lx : s;
+    return ly == 0 ? lx : s;
 }
 
 __device__ inline uint64_t pack(uint32_t kind, uint32_t steps, int32_t value) {
@@ -75,140 +73,168 @@ __device__ inline uint64_t hop(uint64_t e, uint64_t f) {
     return pack(k, s, value_of(f));
 }
 
-// Inlined: as a call its frame spilled to scratch and its registers set the
-// kernel's occupancy.
-__device__ __forceinline__ void trace_tile(uint64_t* L, const int8_t* __restrict__ fd,
+// Pointer of a cell within its tile: kind (2 bits) | steps (16 bits,
+// saturated: a path of more than 4096 is a cycle) | LDS offset of a cell (14
+// bits), K_LOCAL the cell its path has reached, else the cell where it ends.
+constexpr uint32_t P_STEP1 = 1u << 14, P_STEPS = 0xffffu << 14, P_CELL = 0x3fffu;
+__device__ inline uint32_t pointer(uint32_t kind, uint32_t steps, int cell) {
+    return kind << 30 | steps << 14 | (uint32_t)cell << 2;
+}
+// Label of an exit cell between steps 1 and 3: a positive code, the cell it
+// exits from and the steps to that cell (final labels are -stream ids, the
+// negative constants, or 0).
+__device__ inline int32_t exit_code(uint32_t p) { return (int32_t)(p & 0x3fffffffu) - (int32_t)P_STEP1 + 1; }
+__device__ inline int exit_cell(int32_t code) { return ((code - 1) & (int32_t)P_CELL) >> 2; }
+__device__ inline int exit_slot(int32_t code) {
+    return border_slot(exit_cell(code) % TILE, exit_cell(code) / TILE);
+}
+__device__ inline uint32_t exit_steps(int32_t code) { return (uint32_t)(code - 1) / P_STEP1; }
+
+// The tile pass of one tile.  A thread's 16 pointers stay in registers and
+// the tile's in LDS (L), a word a cell.  Bound by its instructions, some 200
+// a cell, and on a grid too small to fill the device by its three rounds of
+// loads.  With 64-bit entries in LDS that carried the labels, read and
+// tested one at a time, loads behind branches (each waited for by itself)
+// and a 64-bit entry a cell for the exits in memory, the launch took 32 us
+// at 1000 x 777 and 148 at 4096^2; now 12 and 68.
+__device__ __forceinline__ void trace_tile(uint32_t* L, const int8_t* __restrict__ fd,
                                            const uint8_t* __restrict__ sf,
                                            const int32_t* __restrict__ slabel,
-                                           uint64_t* __restrict__ ent, int32_t* __restrict__ lab,
-                                           uint64_t* __restrict__ bent, int W, int H, int ntx,
-                                           int t) {
-    const int x0 = (t % ntx) * TILE, y0 = (t / ntx) * TILE;
+                                           int32_t* __restrict__ lab, uint64_t* __restrict__ bent,
+                                           int W, int H, int ntx, int t) {
+    const int tx = t % ntx, ty = t / ntx;
+    const int x0 = tx * TILE, y0 = ty * TILE;
     const int lx = threadIdx.x & 63, strip = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int gx = x0 + lx;
+    const char2* dirs = reinterpret_cast<const char2*>(fd);
 
     // The strip's cells' flags and directions are loaded together, then
-    // their targets' flags and labels: two dependent rounds of loads for the
-    // tile (no load waits on a test; a target outside the grid reads the
-    // cell itself, unused).
-    uint32_t local = 0;
-    constexpr int HALF = STRIP;  // rows per round of loads: all of the strip
-#pragma unroll
-    for (int k0 = 0; k0 < STRIP; k0 += HALF) {
-        uint8_t sfc[HALF], sfn[HALF];
-        char2 dv[HALF];
-        int32_t sln[HALF];
-#pragma unroll
-        for (int j = 0; j < HALF; ++j) {
-            const int gy = y0 + strip * STRIP + k0 + j;
-            sfc[j] = 0;
-            dv[j] = make_char2(0, 0);
-            if (gx < W && gy < H) {
-                const size_t i = (size_t)gy * W + gx;
-                sfc[j] = sf[i];
-                dv[j] = reinterpret_cast<const char2*>(fd)[i];
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < HALF; ++j) {
-            const int gy = y0 + strip * STRIP + k0 + j;
-            const int nx = gx + dv[j].x, ny = gy + dv[j].y;
-            const bool in = gx < W && gy < H && nx >= 0 && ny >= 0 && nx < W && ny < H;
-            const size_t ni = in ? (size_t)ny * W + nx : 0;
-            sfn[j] = 0;
-            sln[j] = 0;
-            if (in) {
-                sfn[j] = sf[ni];
-                sln[j] = slabel[ni];
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < HALF; ++j) {
-            const int k = k0 + j;
-            const int ly = strip * STRIP + k;
-            const int gy = y0 + ly;
-            uint64_t e = pack(K_STUCK, 0, 0);
-            if (gx < W && gy < H) {
-                const char2 d = dv[j];
-                const int nx = gx + d.x, ny = gy + d.y;
-                if (sfc[j] & SF_TRACE) {
-                    e = pack(K_RESOLVED, 0, CAGEO_FLOWTRACE_LAKE);
-                } else if (nx < 0 || ny < 0 || nx >= W || ny >= H) {
-                    e = pack(K_RESOLVED, 1, CAGEO_FLOWTRACE_OUTSIDE);
-                } else if (sfn[j] & SF_TRACE) {
-                    e = pack(K_RESOLVED, 1, sln[j]);
-                } else if (d.x == 0 && d.y == 0) {
-                    e = pack(K_STUCK, 0, 0);
-                } else if (nx >= x0 && ny >= y0 && nx < x0 + TILE && ny < y0 + TILE) {
-                    e = pack(K_LOCAL, 1, (ny - y0) * TILE + (nx - x0));
-                    local |= 1u << k;
-                } else {
-                    e = pack(K_EXIT, 1, (int32_t)((size_t)ny * W + nx));
-                }
-            }
-            L[ly * TILE + lx] = e;
-        }
-    }
-    __syncthreads();
-
-    // Doubling rounds in place: a cell's entry is written by its own thread
-    // only, and the target entry it reads is either last round's or already
-    // this round's, both exact summaries of the target's path.  So every
-    // entry at least doubles its hops a round (paths inside a tile resolve
-    // within 13), step counts stay exact sums, and one barrier a round
-    // suffices.  Entries are 64-bit LDS words, each read or written whole.
-    for (int round = 0; round < 13; ++round) {
-        if (!__syncthreads_or(local != 0)) break;
+    // their targets' flags, then the labels of the targets on a stream.  No
+    // load is conditional (one that is not wanted reads cell 0).  Cells are
+    // numbered in 32 bits (a raster has fewer than 2^31).
+    uint32_t e[STRIP];
+    int32_t val[STRIP];  // of a cell where paths end: its label
+    {
+        const uint32_t first = (uint32_t)(y0 + strip * STRIP) * (uint32_t)W + (uint32_t)gx;
+        const int rows = gx < W ? min(STRIP, H - (y0 + strip * STRIP)) : 0;
+        uint8_t sfc[STRIP], sfn[STRIP];
+        char2 dv[STRIP];
+        uint32_t to[STRIP];
+        uint32_t to_in = 0;  // cells in the grid whose target is
 #pragma unroll
         for (int k = 0; k < STRIP; ++k) {
-            if (local & (1u << k)) {
-                const int li = (strip * STRIP + k) * TILE + lx;
-                const uint64_t e = L[li];
-                const uint64_t nv = hop(e, L[value_of(e)]);
-                L[li] = nv;
-                if (kind_of(nv) != K_LOCAL) local &= ~(1u << k);
-            }
+            const uint32_t i = k < rows ? first + (uint32_t)k * (uint32_t)W : 0u;
+            sfc[k] = sf[i];
+            dv[k] = dirs[i];
+        }
+#pragma unroll
+        for (int k = 0; k < STRIP; ++k) {
+            const int nx = gx + dv[k].x, ny = y0 + strip * STRIP + k + dv[k].y;
+            const bool c = k < rows && (uint32_t)nx < (uint32_t)W && (uint32_t)ny < (uint32_t)H;
+            to[k] = c ? (uint32_t)ny * (uint32_t)W + (uint32_t)nx : 0u;
+            sfn[k] = sf[to[k]];
+            to_in |= (uint32_t)c << k;
+        }
+#pragma unroll
+        for (int k = 0; k < STRIP; ++k) {
+            const bool c = ((to_in >> k) & 1u) && (sfn[k] & SF_TRACE);
+            val[k] = slabel[c ? to[k] : 0u];
+        }
+#pragma unroll
+        for (int k = 0; k < STRIP; ++k) {
+            const int ly = strip * STRIP + k;
+            const int li = ly * TILE + lx;
+            const int dx = dv[k].x, dy = dv[k].y;
+            const bool here = (uint32_t)(lx + dx) < (uint32_t)TILE && (uint32_t)(ly + dy) < (uint32_t)TILE;
+            // the first that holds of: outside the grid, stream, off the
+            // grid, onto a stream, no direction, in the tile, exit (a step
+            // of more than one cell does not join borders: no path)
+            uint32_t p = dx * dx + dy * dy <= 2 ? pointer(K_EXIT, 1, li) : pointer(K_STUCK, 0, li);
+            p = here ? pointer(K_LOCAL, 1, li + dy * TILE + dx) : p;
+            p = (dx | dy) == 0 ? pointer(K_STUCK, 0, li) : p;
+            int32_t v = val[k];
+            p = (sfn[k] & SF_TRACE) ? pointer(K_RESOLVED, 1, li) : p;
+            const bool off = !((to_in >> k) & 1u);
+            p = off ? pointer(K_RESOLVED, 1, li) : p;
+            v = off ? CAGEO_FLOWTRACE_OUTSIDE : v;
+            const bool lake = (sfc[k] & SF_TRACE) != 0;
+            p = lake ? pointer(K_RESOLVED, 0, li) : p;
+            v = lake ? CAGEO_FLOWTRACE_LAKE : v;
+            p = k < rows ? p : pointer(K_STUCK, 0, li);
+            e[k] = p;
+            val[k] = v;
+            L[li] = p;
         }
     }
     __syncthreads();
-    // Outputs: the labels of the cells whose path ends in the tile; for an
-    // exit cell, the border slot it exits to (in the entry raster) and the
-    // mark EXIT_MARK; the tile's border table, every slot written (cells
-    // outside the grid and the four unused slots stuck).
-    uint64_t* tb = bent + (size_t)t * BORDER_SLOTS;
+    const char* Lb = reinterpret_cast<const char*>(L);
+    auto at = [&](uint32_t p) { return *reinterpret_cast<const uint32_t*>(Lb + (p & P_CELL)); };
+
+    // Doubling rounds in place: a cell's pointer is written by its own
+    // thread only, and the target's that it reads is either last round's or
+    // already this round's, both exact summaries of the target's path.  So
+    // every pointer at least doubles its hops a round (paths inside a tile
+    // resolve within 13), step counts stay exact sums, and one barrier a
+    // round suffices.
+    for (int round = 0; round < 13; ++round) {
+        uint32_t p[STRIP];
+        uint32_t all = 0xffffffffu;
+#pragma unroll
+        for (int k = 0; k < STRIP; ++k) p[k] = at(e[k]);
+#pragma unroll
+        for (int k = 0; k < STRIP; ++k) {
+            const uint32_t s = min((e[k] & P_STEPS) + (p[k] & P_STEPS), P_STEPS);
+            const uint32_t n = (p[k] & ~P_STEPS) | s;
+            e[k] = e[k] >> 30 == K_LOCAL ? n : e[k];
+            L[(strip * STRIP + k) * TILE + lx] = e[k];
+            all = min(all, e[k]);
+        }
+        static_assert(K_LOCAL == 0, "the least kind");
+        if (!__syncthreads_or(all >> 30 == K_LOCAL)) break;
+    }
+    // The border cells, one a thread in the order of the slots: wave 0 the
+    // first row, 1 the last, 2 the first column, 3 the last (rows 1 to 62;
+    // the other four threads' slots are unused).
+    const int bx = strip < 2 ? lx : strip == 2 ? 0 : TILE - 1;
+    const int by = strip == 0 ? 0 : strip == 1 ? TILE - 1 : lx;
+    const bool used = strip < 2 || (lx > 0 && lx < TILE - 1);
+    const uint32_t bp = L[by * TILE + bx];
+    int32_t slot = 0;  // that an exit leads to
+    if (bp >> 30 == K_EXIT) {
+        const int end = (int)((bp & P_CELL) >> 2);
+        const uint32_t ex = (uint32_t)(x0 + end % TILE), ey = (uint32_t)(y0 + end / TILE);
+        const char2 d = dirs[ey * (uint32_t)W + ex];
+        const uint32_t nx = ex + (uint32_t)(int)d.x, ny = ey + (uint32_t)(int)d.y;
+        slot = (int)((ny / TILE) * (uint32_t)ntx + nx / TILE) * BORDER_SLOTS +
+               border_slot((int)(nx % TILE), (int)(ny % TILE));
+    }
+    __syncthreads();
+    // Where paths end, the cell's label takes the pointer's place.
 #pragma unroll
     for (int k = 0; k < STRIP; ++k) {
-        const int ly = strip * STRIP + k;
-        const int gy = y0 + ly;
-        uint64_t e = pack(K_STUCK, 0, 0);
-        if (gx < W && gy < H) {
-            e = L[ly * TILE + lx];
-            const uint32_t kind = kind_of(e);
-            const size_t i = (size_t)gy * W + gx;
-            int32_t label = 0;
-            if (kind == K_RESOLVED) {
-                label = value_of(e);
-            } else if (kind == K_EXIT) {
-                // the first cell outside the tile: a border cell of the next tile
-                const uint32_t ti = (uint32_t)value_of(e);
-                const int ny = (int)(ti / (uint32_t)W), nx = (int)(ti - (uint32_t)ny * W);
-                const int slot = ((ny / TILE) * ntx + nx / TILE) * BORDER_SLOTS +
-                                 border_slot(nx % TILE, ny % TILE);
-                e = pack(K_EXIT, steps_of(e), slot);
-                ent[i] = e;
-                label = EXIT_MARK;
-            } else {
-                e = pack(K_STUCK, 0, 0);  // K_LOCAL: a cycle inside the tile
-            }
-            lab[i] = label;
-        }
-        const int slot = border_slot(lx, ly);
-        if (slot >= 0) tb[slot] = e;
+        const int li = (strip * STRIP + k) * TILE + lx;
+        if ((e[k] & P_CELL) == (uint32_t)li << 2) L[li] = (uint32_t)val[k];
     }
-    if (threadIdx.x < 4)
-        tb[threadIdx.x < 2 ? 2 * TILE + (TILE - 1) * threadIdx.x
-                           : 3 * TILE + (TILE - 1) * (threadIdx.x - 2)] = pack(K_STUCK, 0, 0);
     __syncthreads();
+    // Outputs: labels and exit codes; the tile's border table, every slot
+    // written (cells outside the grid and the four unused slots stuck).
+    {
+        const uint32_t kind = bp >> 30, steps = (bp & P_STEPS) / P_STEP1;
+        uint64_t f = pack(K_STUCK, 0, 0);
+        if (used && kind == K_RESOLVED) f = pack(K_RESOLVED, steps, (int32_t)at(bp));
+        if (used && kind == K_EXIT) f = pack(K_EXIT, steps, slot);
+        bent[(size_t)t * BORDER_SLOTS + threadIdx.x] = f;
+    }
+    int32_t* out = lab + (size_t)(y0 + strip * STRIP) * W + x0;
+    const int rows = gx < W ? min(STRIP, H - (y0 + strip * STRIP)) : 0;
+#pragma unroll
+    for (int k = 0; k < STRIP; ++k) {
+        const uint32_t kind = e[k] >> 30;
+        int32_t label = (int32_t)at(e[k]);
+        label = kind == K_RESOLVED ? label : 0;  // (K_LOCAL: a cycle inside the tile)
+        label = kind == K_EXIT ? exit_code(e[k]) : label;
+        if (k < rows) out[(size_t)k * W + lx] = label;
+    }
 }
 
 
@@ -229,7 +255,6 @@ struct TrRaster {
     const int8_t* fd;
     const uint8_t* sf;
     const int32_t* slabel;
-    uint64_t* ent;  // one 64-bit entry per cell (written for exit cells)
     uint64_t* bent; // border table: BORDER_SLOTS entries per tile
     int32_t* lab;
     int W, H, ntx;
@@ -269,8 +294,8 @@ __device__ inline TrBlock tr_block(const TrArgs& a, int g) {
 // Final label of cell 0 of a raster (between steps 2 and 3 of the launch).
 __device__ inline int32_t label_of_cell0(const TrRaster& R) {
     const int32_t v = R.lab[0];
-    if (v != EXIT_MARK) return v;
-    const uint64_t f = ld64(&R.bent[value_of(R.ent[0])]);
+    if (v <= 0) return v;
+    const uint64_t f = ld64(&R.bent[exit_slot(v)]);  // block 0's
     return kind_of(f) == K_RESOLVED ? value_of(f) : 0;
 }
 
@@ -290,12 +315,12 @@ __device__ inline uint32_t* tr_rounds(const TrArgs& a, uint32_t group) {
 // boundary orders that before their first use.
 template <bool MULTI>
 __global__ __launch_bounds__(256) void k_tr_tiles(TrArgs a) {
-    __shared__ uint64_t L[TILE * TILE];
+    __shared__ uint32_t L[TILE * TILE];
     const TrBlock b = tr_block<MULTI>(a, blockIdx.x);
     const TrRaster& R = b.R;
     if (b.lb == 0 && threadIdx.x == 0) R.scal[SC_LONGPATH] = 0;
     if (blockIdx.x == 0 && threadIdx.x < CTL_PF_GROUPS) *tr_rounds(a, threadIdx.x) = 0u;
-    trace_tile(L, R.fd, R.sf, R.slabel, R.ent, R.lab, R.bent, R.W, R.H, R.ntx, b.lb);
+    trace_tile(L, R.fd, R.sf, R.slabel, R.lab, R.bent, R.W, R.H, R.ntx, b.lb);
 }
 
 // Jumping over the border tables: thread s takes slot s % BORDER_SLOTS of
@@ -338,13 +363,14 @@ __global__ __launch_bounds__(256) void k_tr_jump(TrArgs a) {
 }
 
 // Exit cells take their slot's label; performConnectFlowPath maps a label 0
-// to label[0] when that is negative.  An exit whose chain is still moving
-// (a cycle through tiles) or ends stuck stays 0.  One workgroup per block,
-// a wave per strip of STRIP rows (one lane per column): the strip's labels,
-// then its exit cells' entries, then their slots' entries, each round of
-// loads issued whole before the next.
+// to label[0] when that is negative.  An exit whose chain is a cycle through
+// tiles or ends stuck stays 0.  One workgroup per block, its border table in
+// LDS, a wave per strip of STRIP rows (one lane per column).  One round of
+// loads, where a 64-bit entry a cell and its slot's from another tile made
+// it three: 23 us at 4096^2, 45 before.
 template <bool MULTI>
 __global__ __launch_bounds__(256) void k_tr_exits(TrArgs a) {
+    __shared__ uint64_t tb[BORDER_SLOTS];
     if (blockIdx.x == 0 && threadIdx.x < CTL_PF_GROUPS) {
         uint32_t r = ld(tr_rounds(a, threadIdx.x));
         for (int off = 32; off > 0; off >>= 1) r = max(r, (uint32_t)__shfl_xor((int)r, off));
@@ -355,27 +381,25 @@ __global__ __launch_bounds__(256) void k_tr_exits(TrArgs a) {
     const int x = (b.lb % R.ntx) * TILE + (threadIdx.x & 63);
     const int y0 = (b.lb / R.ntx) * TILE + (int)(threadIdx.x >> 6) * STRIP;
     const int rows = x < R.W ? min(STRIP, R.H - y0) : 0;
-    const int32_t l0 = label_of_cell0(R);
+    static_assert(BORDER_SLOTS == TILE_THREADS, "a slot a thread");
+    const uint64_t own = R.bent[(size_t)b.lb * BORDER_SLOTS + threadIdx.x];
     int32_t v[STRIP];
 #pragma unroll
-    for (int k = 0; k < STRIP; ++k) v[k] = k < rows ? R.lab[(size_t)(y0 + k) * R.W + x] : 1;
-    uint64_t e[STRIP];
-#pragma unroll
-    for (int k = 0; k < STRIP; ++k)
-        e[k] = v[k] == EXIT_MARK ? R.ent[(size_t)(y0 + k) * R.W + x] : 0;
-    uint64_t f[STRIP];
-#pragma unroll
-    for (int k = 0; k < STRIP; ++k) f[k] = v[k] == EXIT_MARK ? ld64(&R.bent[value_of(e[k])]) : 0;
+    for (int k = 0; k < STRIP; ++k) v[k] = k < rows ? R.lab[(size_t)(y0 + k) * R.W + x] : -1;
+    const int32_t l0 = label_of_cell0(R);
+    tb[threadIdx.x] = own;
+    __syncthreads();
     uint32_t longp = 0;
 #pragma unroll
     for (int k = 0; k < STRIP; ++k) {
-        if (k >= rows) continue;
         int32_t w = v[k];
-        if (w == EXIT_MARK) {
+        if (w > 0) {
+            const uint64_t f = tb[exit_slot(w)];
+            const uint32_t steps = exit_steps(w) + steps_of(f);
             w = 0;
-            if (kind_of(f[k]) == K_RESOLVED) {
-                w = value_of(f[k]);
-                if (steps_of(e[k]) + steps_of(f[k]) > 100001u) ++longp;  // past the walk guard
+            if (kind_of(f) == K_RESOLVED) {
+                w = value_of(f);
+                if (steps > 100001u) ++longp;  // past the walk guard
             }
         }
         if (w == 0 && l0 < 0) w = l0;
@@ -407,7 +431,6 @@ TrRaster tr_raster(Context* c, const int8_t* fd, const uint8_t* sflags, const in
     R.fd = fd;
     R.sf = sflags;
     R.slabel = slabel;
-    R.ent = c->d_ptr;
     R.bent = c->d_bent;
     R.lab = lab;
     R.W = c->W;
@@ -419,8 +442,7 @@ TrRaster tr_raster(Context* c, const int8_t* fd, const uint8_t* sflags, const in
 
 }  // namespace
 
-// Needs one 64-bit raster, c->d_ptr.  The long-path count is
-// left in the scalar block.
+// The long-path count is left in the scalar block.
 int flow_tracing_grid_cap(Context* c, int* cap) {
     return jump_cap(reinterpret_cast<const void*>(k_tr_jump<false>), c->device, cap);
 }
