@@ -112,43 +112,59 @@ __device__ inline uint32_t ld(const uint32_t* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// s / 1.41421356237309505f for s in [2^-77, 2^100), correctly rounded:
+// Markstein's correction of a quotient by its exact remainder (equal to the
+// division for every significand), three instructions where the division
+// takes eleven.
+constexpr float DIAGONAL = 1.41421356237309505f;
+constexpr float DIV_LOW = 0x1p-77f, DIV_HIGH = 0x1p100f;
+__device__ inline float over_diagonal(float s) {
+    constexpr float y = 1.0f / DIAGONAL;
+    const float q = s * y;
+    return __builtin_fmaf(__builtin_fmaf(-q, DIAGONAL, s), y, q);
+}
+
 // D8 of one cell (FlowRoutingAlgorithmCPUOpenMP.h:60-150) at grid position
 // (x, y), its elevation zc and its neighbours' nb.  Returns the initial
-// distance: 0 has a direction, D_STREAM, or D_INF (flat); (ox, oy) the
-// direction.  Edge cells point out of the grid and read no neighbour, so
-// values outside the grid are never used.
-__device__ inline int32_t d8_of(float zc, const float* nb, int x, int y, int W, int H, int8_t& ox,
-                                int8_t& oy) {
-    int dxi = 0, dyi = 0;
-    if (x == 0) dxi = -1;
-    else if (x == W - 1) dxi = 1;
-    if (y == 0) dyi = -1;
-    else if (y == H - 1) dyi = 1;
-    ox = 0;
-    oy = 0;
-    if (dxi != 0 || dyi != 0) {
-        ox = (int8_t)dxi;
-        oy = (int8_t)dyi;
-        return 0;
-    }
-    if (zc == 0.0f) return D_STREAM;
-    // the direction is carried as its offsets, each a constant of the
-    // unrolled loop (indexing the tables by a variable would load them from
-    // memory)
-    float steepest = 0.0f;
-    int32_t d = D_INF;
+// distance: 0 has a direction, D_STREAM, or D_INF (flat); `dir` the
+// direction, x offset in the low byte and y offset in the next.  Edge cells
+// point out of the grid and read no neighbour, so values outside the grid
+// are never used.  Without branches but for drops outside the range of
+// over_diagonal (a test and a division behind it for each neighbour took the
+// launch 38 us at 1000 x 777 and 157 at 4096^2; now 34 and 143).
+__device__ inline int32_t d8_of(float zc, const float* nb, int x, int y, int W, int H,
+                                uint32_t& dir) {
+    float s[8], steepest = 0.0f, most = 0.0f;
+    uint32_t least = 0xffffffffu;  // of the positive diagonal drops, less one
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
-        float s = zc - nb[k];
-        if (s > 0.0f) {
-            if (k & 1) s = s / 1.41421356237309505f;
-            if (s > steepest) {
-                steepest = s;
-                ox = (int8_t)FDX[k];
-                oy = (int8_t)FDY[k];
-                d = 0;
-            }
+        s[k] = fmaxf(zc - nb[k], 0.0f);  // (0 for a NaN)
+        if (k & 1) {
+            most = fmaxf(most, s[k]);
+            least = min(least, __float_as_uint(s[k]) - 1u);
         }
+    }
+    if (most >= DIV_HIGH || least < __float_as_uint(DIV_LOW) - 1u) {
+#pragma unroll
+        for (int k = 1; k < 8; k += 2) s[k] = s[k] / DIAGONAL;
+    } else {
+#pragma unroll
+        for (int k = 1; k < 8; k += 2) s[k] = over_diagonal(s[k]);
+    }
+    dir = 0;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const uint32_t code = (uint32_t)(uint8_t)FDX[k] | (uint32_t)(uint8_t)FDY[k] << 8;
+        dir = s[k] > steepest ? code : dir;
+        steepest = fmaxf(steepest, s[k]);
+    }
+    int32_t d = steepest > 0.0f ? 0 : D_INF;
+    d = zc == 0.0f ? D_STREAM : d;
+    dir = zc == 0.0f ? 0u : dir;
+    const int dxi = x == 0 ? -1 : x == W - 1 ? 1 : 0, dyi = y == 0 ? -1 : y == H - 1 ? 1 : 0;
+    if ((dxi | dyi) != 0) {
+        d = 0;
+        dir = (uint32_t)(uint8_t)dxi | (uint32_t)(uint8_t)dyi << 8;
     }
     return d;
 }
@@ -167,6 +183,9 @@ __device__ inline Row64 row_read(Row64 v, int lane) {
     const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, lane);
     const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), lane);
     return ((Row64)hi << 32) | lo;
+}
+__device__ inline void row_write(Row64& v, Row64 x, int lane) {
+    v = (int)(threadIdx.x & 63) == lane ? x : v;
 }
 __device__ inline int wave_min(int v) {
     int none = 0;
@@ -226,7 +245,7 @@ __device__ inline void ring_offers(Levels& v, const int* d) {
 // it; the step numbers are recorded in bit planes because a store a cell
 // would cost the fullest row's cells one after the other.  Sweeps of row
 // solves (min-plus scans along each row, four waves a tile) did the same
-// work before: the D8 kernel took 81 us at 1000 x 777 and 313 at 4096^2, now
+// work before: the D8 kernel took 81 us at 1000 x 777 and 313 at 4096^2, then
 // 38 and 157; the passes 117 and 379, now 87 and 307 (a grid barrier a
 // pass, some 8 to 13 us, is most of what is left of them).
 __device__ inline void flat_levels(Levels& v, FrTile& T, FrSolve& S) {
@@ -424,11 +443,8 @@ __device__ void bfs_tile(FrTile& T, FrSolve& S, const FrArgs& args, const FrBloc
 #pragma unroll
     for (int k = 0; k < STRIP; ++k) {
         const int d = T.d[(strip * STRIP + k + 1) * HALO_W + lx + 1];
-        const Row64 i = __ballot(d == D_INF), f = __ballot(d >= 1 && d < D_INF);
-        if (lx == k) {
-            inf = i;
-            fin = f;
-        }
+        row_write(inf, __ballot(d == D_INF), k);
+        row_write(fin, __ballot(d >= 1 && d < D_INF), k);
     }
     if (lx < STRIP) {
         T.inf[strip * STRIP + lx] = inf;
@@ -516,8 +532,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
             float nb[8];
 #pragma unroll
             for (int q = 0; q < 8; ++q) nb[q] = U.zt[c + FDY[q] * ZW + FDX[q]];
-            int8_t ox, oy;
-            d = d8_of(U.zt[c], nb, gx, gy, R.W, R.H, ox, oy);
+            uint32_t dir;
+            d = d8_of(U.zt[c], nb, gx, gy, R.W, R.H, dir);
         }
         T.d[hy * HALO_W + hx] = d;
     }
@@ -541,24 +557,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
 #pragma unroll
             for (int j = 0; j < 3; ++j) dn[j] = col[(k + 2) * ZW + j];
             const float nb[8] = {up[1], up[2], at[2], dn[2], dn[1], dn[0], at[0], up[0]};
-            int d = D_OUT;
-            if (gx < R.W && gy < R.H) {
-                int8_t ox, oy;
-                d = d8_of(at[1], nb, gx, gy, R.W, R.H, ox, oy);
-                reinterpret_cast<char2*>(R.fd)[(size_t)gy * R.W + gx] = make_char2(ox, oy);
-            }
+            uint32_t dir;
+            int d = d8_of(at[1], nb, gx, gy, R.W, R.H, dir);
+            if (gx < R.W && gy < R.H)
+                reinterpret_cast<uint16_t*>(R.fd)[(size_t)gy * R.W + gx] = (uint16_t)dir;
+            else
+                d = D_OUT;
             T.d[(ly + 1) * HALO_W + lx + 1] = d;
-            const Row64 flat = __ballot(d == D_INF), has = __ballot(d == 0);
-            if (lx == k) {
-                inf = flat;
-                zero = has;
-            }
+            const Row64 flat = __ballot(d == D_INF);
+            row_write(inf, flat, k);
+            row_write(zero, __ballot(d == 0), k);
             if (flat) {
 #pragma unroll
-                for (int q = 0; q < 8; ++q) {
-                    const Row64 m = __ballot(d == D_INF && nb[q] <= at[1]);
-                    if (lx == k) nbr[q] = m;
-                }
+                for (int q = 0; q < 8; ++q)
+                    row_write(nbr[q], flat & __ballot(nb[q] <= at[1]), k);
             }
 #pragma unroll
             for (int j = 0; j < 3; ++j) {

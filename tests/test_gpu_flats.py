@@ -70,3 +70,23 @@ def test_lakes_across_tiles(ca, torch_cuda, seed):
         z[r.integers(2, h - 2), r.integers(2, w - 2)] = 1.5
     z[r.integers(2, h - 2), r.integers(2, w - 2)] = 0.0
     route(ca, torch_cuda, z)
+
+
+@pytest.mark.parametrize("seed", range(3))
+def test_drop_ranges(ca, torch_cuda, seed):
+    """Drops of every magnitude, denormal to infinite, and diagonal drops about
+    the square root of two times the straight ones."""
+    announce("drops", seed)
+    r = np.random.default_rng(seed)
+    h, w = 131, 190
+    z = np.float32(10.0) ** r.uniform(-44, 38, (h, w)).astype(np.float32)
+    z[r.random((h, w)) < 0.02] = np.inf
+    z[r.random((h, w)) < 0.02] = 0.0
+    near = np.float32(100.0) - np.float32(0.001) * r.integers(0, 4000, (h, w)).astype(np.float32)
+    step = np.where((np.add.outer(np.arange(h), np.arange(w)) & 1) == 0, np.float32(1.0),
+                    np.float32(1.4142135))
+    ties = (np.float32(7.0) - step * r.integers(0, 2, (h, w)).astype(np.float32) -
+            r.integers(0, 3, (h, w)).astype(np.float32) * np.float32(2.0 ** -22))
+    with np.errstate(all="ignore"):
+        for g in (z, near, ties.astype(np.float32)):
+            route(ca, torch_cuda, g)
