@@ -44,7 +44,7 @@ int alloc(T** p, size_t count) {
 
 void free_all(Context* c) {
     void* ptrs[] = {c->d_mark, c->d_xb, c->d_pfmask, c->d_pfinfo, c->d_rows, c->d_work3, c->d_ctrl, c->d_bar, c->d_scal, c->d_bmm, c->d_filter,
-                    c->d_sflags, c->d_slabel, c->d_off, c->d_factor, c->d_a, c->d_b, c->d_z,
+                    c->d_sflags, c->d_slabel, c->d_factor, c->d_a, c->d_b, c->d_z,
                     c->d_w, c->d_st, c->d_fd, c->d_dist, c->d_lab, c->d_ptr, c->d_bent,
                     c->d_lr_col, c->d_lr_row, c->d_lr_planes};
     for (void* p : ptrs)
@@ -247,7 +247,6 @@ int cageo_context_create(cageo_context** out, int W, int H, void* stream) {
     A(cageo::alloc(&c->d_sflags, n));
     A(cageo::alloc(&c->d_slabel, n));
     const int maxoff = (2 * CAGEO_MAX_BEVEL_RADIUS + 1) * (2 * CAGEO_MAX_BEVEL_RADIUS + 1);
-    A(cageo::alloc(&c->d_off, 2 * maxoff));
     A(cageo::alloc(&c->d_factor, maxoff));
     A(cageo::alloc(&c->d_a, n));
     A(cageo::alloc(&c->d_b, n));

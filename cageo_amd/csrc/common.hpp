@@ -103,7 +103,6 @@ struct Context {
 
     // burn offsets (x, y, factor), ordered as the reference's search array
     int n_offsets = 0;
-    int* d_off = nullptr;      // 2 ints per offset
     float* d_factor = nullptr;  // one factor per offset
     int off_radius = -1;
 

@@ -20,6 +20,7 @@
 // unburned values.
 #include <cmath>
 #include <list>
+#include <type_traits>
 #include <vector>
 
 #include "tiles.hpp"
@@ -59,37 +60,42 @@ __global__ __launch_bounds__(256) void k_realistic(const float* __restrict__ dem
         field[i] = realistic_value(dem[i], field[i], nodata);
 }
 
-// Burning works on LDS tiles of 64 x 16 cells with an R-cell halo holding
-// the unburned values and, per cell, the two facts the search asks about a
-// neighbour n, given that n is in the grid and a stream cell:
-//   BF_BURN  n is a stream cell;
-//   BF_LATE  n is a stream cell whose unburned value is not nodata_dem.
+// Burning works on blocks of 64 x 32 cells, a wave for 8 rows of them.  What
+// the search asks about a neighbour n is one of two facts, given that n is in
+// the grid:
+//   burn  n is a stream cell;
+//   late  n is a stream cell whose unburned value is not nodata_dem.
 // A neighbour that precedes the cell in raster order (offset dy < 0, or
 // dy == 0 and dx < 0: for in-grid cells the reference's n < i reduces to
 // the offset alone) has been burned to 0 already and qualifies when
-// 0 != nodata_dem, i.e. by BF_BURN under that launch constant; a later one
-// qualifies by BF_LATE.  Halo cells outside the grid hold no flag, which
-// is the reference's in-grid test.  Each offset's LDS step and the flag it
-// needs are packed into one word of a table staged in LDS.
-constexpr int BT_X = 64, BT_Y = 16;
+// 0 != nodata_dem, i.e. by `burn` under that launch constant; a later one
+// qualifies by `late`.  Both are kept as bit masks, a window of 64 + 2R cells
+// a row (cells outside the grid have no bit, which is the reference's in-grid
+// test): a cell's neighbourhood is then 2R + 1 bits of each of 2R + 1 words,
+// and a distance's offsets are tested together, their factor being the same.
+// Bound by its loads, all of them issued before the first is used.  A byte
+// of flags a cell in LDS, read offset by offset, took 145 us at 4096^2 and
+// 547 at 8192^2 (with the minimum and maximum); now 73 and 241 (a copy of as
+// many bytes: 42 and 168).  Shifting uniform words offset by offset in scalar
+// registers was slower, 169 and 613: a serial chain for each row.
+constexpr int BT_X = 64, BT_R = 8, BT_Y = 4 * BT_R;
 constexpr int BH_MAX = CAGEO_MAX_BEVEL_RADIUS;
-constexpr int BL_W = BT_X + 2 * BH_MAX, BL_H = BT_Y + 2 * BH_MAX;
-constexpr int BOFF_MAX = (2 * BH_MAX + 1) * (2 * BH_MAX + 1);
-constexpr uint8_t BF_BURN = 1, BF_LATE = 2;
+constexpr int BE_Y = BT_Y + 2 * BH_MAX;  // rows of a block with its halo
+static_assert(BH_MAX <= 8, "the 2R side cells of a row take 16 bits");
+static_assert(BT_R + 2 * BH_MAX <= 64, "a row of a wave's windows a lane");
+typedef unsigned long long Mask64;
 
 // REAL: the tile's values are realistic_value(z0, z1) (the fused Monte
-// Carlo pass), else z0 itself.
-template <bool REAL>
+// Carlo pass), else z0 itself.  out[j]: burned value of column gx, row gy + j.
+template <bool REAL, int R>
 __device__ inline void burn_tile(int W, int H, const uint8_t* __restrict__ sf,
-                                 const int* __restrict__ off, const float* __restrict__ fac,
-                                 int n_off, int R, float nodata_dem,
+                                 const float* __restrict__ fac, int n_off, float nodata_dem,
                                  const float* __restrict__ z0, const float* __restrict__ z1,
-                                 float out[4], int gx_out[4], int gy_out[4]) {
-    __shared__ float zt[BL_W * BL_H];
-    __shared__ uint8_t ft[BL_W * BL_H];
-    __shared__ int s_step[BOFF_MAX];  // LDS step << 2 | flag the offset needs
-    __shared__ float s_fac[BOFF_MAX];
-    constexpr int ITER = (BL_W * BL_H + 255) / 256;  // loads per thread at the largest radius
+                                 float out[BT_R], int& gx, int& gy) {
+    constexpr int NH = (2 * R + 3) / 4;                          // halo rows of a wave
+    constexpr int NS = R ? (16 * (BT_Y + 2 * R) + 255) / 256 : 0;  // side cells of a thread
+    __shared__ Mask64 s_burn[BE_Y], s_late[BE_Y];  // the 64 cells of the block's columns
+    __shared__ Mask64 s_sburn[NS * 4 + 1], s_slate[NS * 4 + 1];  // side cells, 16 bits a row
     // Blocks go round robin over the 8 XCDs; renumbering them so that each
     // XCD takes a contiguous band of tiles keeps the neighbours whose cache
     // lines hold this tile's halo in the same L2 (a bijection on the block
@@ -98,94 +104,146 @@ __device__ inline void burn_tile(int W, int H, const uint8_t* __restrict__ sf,
     unsigned t = blockIdx.y * gridDim.x + blockIdx.x;
     if ((nb & 7) == 0) t = (t & 7) * (nb >> 3) + (t >> 3);
     const int x0 = (int)(t % gridDim.x) * BT_X, y0 = (int)(t / gridDim.x) * BT_Y;
-    const int lw = BT_X + 2 * R, lh = BT_Y + 2 * R;
-    // All of a thread's loads are issued before any of them is used: a cell
-    // outside the grid or the halo of radius R loads cell 0 (cached) and is
-    // replaced afterwards, so no load sits in a branch that would have to
-    // wait for it.
-    float av[ITER], bv[ITER];
-    uint8_t fv[ITER];
-    bool in[ITER];
+    const int lx = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    gx = x0 + lx;
+    gy = y0 + wave * BT_R;
+    // A cell outside the grid, or beyond the radius, loads cell 0 (cached)
+    // and is replaced afterwards, so no load sits in a branch.
+    struct Cell {
+        float a, b;
+        uint8_t f;
+        bool in;
+    };
+    auto load = [&](int x, int y, bool want) {
+        Cell c;
+        c.in = want && x >= 0 && y >= 0 && x < W && y < H;
+        const size_t i = c.in ? (size_t)y * W + x : 0;
+        c.a = z0[i];
+        c.b = REAL ? z1[i] : 0.0f;
+        c.f = sf[i];
+        return c;
+    };
+    Cell own[BT_R], halo[NH + 1], side[NS + 1];
 #pragma unroll
-    for (int it = 0; it < ITER; ++it) {
-        const int k = threadIdx.x + it * 256;
-        const int ly = k / lw, lx = k - ly * lw;
-        const int gx = x0 - R + lx, gy = y0 - R + ly;
-        in[it] = k < lw * lh && gx >= 0 && gy >= 0 && gx < W && gy < H;
-        const size_t gi = in[it] ? (size_t)gy * W + gx : 0;
-        av[it] = z0[gi];
-        bv[it] = REAL ? z1[gi] : 0.0f;
-        fv[it] = sf[gi];
-    }
-    if ((int)threadIdx.x < n_off) {
-        const int o = threadIdx.x, ox = off[2 * o], oy = off[2 * o + 1];
-        const bool early = oy < 0 || (oy == 0 && ox < 0);
-        const int need = early ? (nodata_dem != 0.0f ? BF_BURN : 0) : BF_LATE;
-        s_step[o] = (oy * BL_W + ox) * 4 + need;
-        s_fac[o] = fac[o];
+    for (int j = 0; j < BT_R; ++j) own[j] = load(gx, gy + j, true);
+#pragma unroll
+    for (int j = 0; j < NH; ++j) {
+        const int k = wave + 4 * j;  // halo row: R above, R below
+        halo[j] = load(gx, k < R ? y0 - R + k : y0 + BT_Y + k - R, k < 2 * R);
     }
 #pragma unroll
-    for (int it = 0; it < ITER; ++it) {
-        const int k = threadIdx.x + it * 256;
-        if (k < lw * lh) {
-            const int ly = k / lw, lx = k - ly * lw;
-            float v = 0.0f;
-            uint8_t f = 0;
-            if (in[it]) {
-                v = REAL ? realistic_value(av[it], bv[it], nodata_dem) : av[it];
-                if (fv[it] & SF_BURN) f = BF_BURN | (v != nodata_dem ? BF_LATE : 0);
-            }
-            zt[ly * BL_W + lx] = v;
-            ft[ly * BL_W + lx] = f;
+    for (int j = 0; j < NS; ++j) {
+        const int i = threadIdx.x + 256 * j, c = i & 15, k = i >> 4;
+        side[j] = load(c < R ? x0 - R + c : x0 + BT_X + c - R, y0 - R + k,
+                       c < 2 * R && k < BT_Y + 2 * R);
+    }
+    auto value = [&](const Cell& c) { return REAL ? realistic_value(c.a, c.b, nodata_dem) : c.a; };
+    auto masks = [&](const Cell& c, float v, Mask64& burn, Mask64& late) {
+        const bool f = c.in && (c.f & SF_BURN);
+        burn = __ballot(f);
+        late = __ballot(f && v != nodata_dem);
+    };
+    Mask64 stream[BT_R];
+#pragma unroll
+    for (int j = 0; j < BT_R; ++j) {
+        Mask64 late;
+        out[j] = value(own[j]);
+        masks(own[j], out[j], stream[j], late);
+        s_burn[R + wave * BT_R + j] = stream[j];
+        s_late[R + wave * BT_R + j] = late;
+        if (own[j].f & SF_BURN) out[j] = 0.0f;
+    }
+#pragma unroll
+    for (int j = 0; j < NH; ++j) {
+        const int k = wave + 4 * j;
+        Mask64 burn, late;
+        masks(halo[j], value(halo[j]), burn, late);
+        if (k < 2 * R) {
+            s_burn[k < R ? k : BT_Y + k] = burn;
+            s_late[k < R ? k : BT_Y + k] = late;
         }
     }
-    __syncthreads();
-    // Each thread's four cells (one column, four rows) search side by side:
-    // per offset one table read and four independent flag reads.  A cell
-    // takes the first offset, in the search array's order, whose cell
-    // qualifies; stream cells become 0.
-    const int lx = threadIdx.x & 63;
-    int c[4];
-    bool done[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int ly = (threadIdx.x >> 6) * 4 + j;
-        gx_out[j] = x0 + lx;
-        gy_out[j] = y0 + ly;
-        c[j] = (ly + R) * BL_W + lx + R;
-        out[j] = zt[c[j]];
-        done[j] = (ft[c[j]] & BF_BURN) != 0;
-        if (done[j]) out[j] = 0.0f;
+    for (int j = 0; j < NS; ++j) {
+        Mask64 burn, late;
+        masks(side[j], value(side[j]), burn, late);
+        s_sburn[4 * j + wave] = burn;
+        s_slate[4 * j + wave] = late;
     }
-    for (int o = 0; o < n_off; ++o) {
-        if (!__any(!(done[0] && done[1] && done[2] && done[3]))) break;
-        const int s = s_step[o];
-        const float f = s_fac[o];
-        uint8_t q[4];
+    __syncthreads();
+    if constexpr (R > 0) {
+        // Row e of the wave's rows with their halo, as each lane sees it: bit
+        // i is column gx + i - R.
+        constexpr int E = BT_R + 2 * R, F = 2 * R + 1;
+        uint32_t fb[E], fl[E];
+        auto field = [&](Mask64 mid, uint32_t s) {
+            const Mask64 lo = mid << R | (s & ((1u << R) - 1u));
+            const Mask64 hi = mid >> (64 - R) | (Mask64)(s >> R) << R;
+            return ((uint32_t)(lo >> lx) | (uint32_t)((hi << 1) << (63 - lx))) & ((1u << F) - 1u);
+        };
+        bool some = false;  // a stream cell in those rows
 #pragma unroll
-        for (int j = 0; j < 4; ++j) q[j] = ft[c[j] + (s >> 2)];
+        for (int e = 0; e < E; ++e) {
+            const int row = wave * BT_R + e;
+            const uint32_t sb = (uint32_t)(s_sburn[row >> 2] >> (16 * (row & 3))) & 0xffffu;
+            const uint32_t sl = (uint32_t)(s_slate[row >> 2] >> (16 * (row & 3))) & 0xffffu;
+            fb[e] = nodata_dem != 0.0f ? field(s_burn[row], sb) : 0u;
+            fl[e] = field(s_late[row], sl);
+            some |= (fb[e] | fl[e]) != 0u;
+        }
+        if (!__any(some)) return;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            if (!done[j] && (q[j] & s & 3)) {
-                out[j] = out[j] * f;
-                done[j] = true;
+        for (int j = 0; j < BT_R; ++j) {
+            if (own[j].f & SF_BURN) continue;
+            // Qualifying neighbours by row.  The search takes the first in
+            // order of distance, and its factor depends on the distance only.
+            uint32_t q[F];
+#pragma unroll
+            for (int d = 0; d < F; ++d) {
+                const uint32_t before = (1u << R) - 1u;
+                q[d] = d < R ? fb[j + d]
+                             : d > R ? fl[j + d] : (fb[j + d] & before) | (fl[j + d] & ~before & ~(1u << R));
             }
+            float f = 1.0f;
+            int o = n_off;
+            bool found = false;
+#pragma unroll
+            for (int d2 = R * R; d2 >= 1; --d2) {  // (the nearest is written last)
+                int count = 0;
+                uint32_t any = 0;
+#pragma unroll
+                for (int d = 0; d < F; ++d) {
+                    uint32_t m = 0;
+#pragma unroll
+                    for (int i = 0; i < F; ++i)
+                        if ((i - R) * (i - R) + (d - R) * (d - R) == d2) {
+                            m |= 1u << i;
+                            ++count;
+                        }
+                    any |= q[d] & m;
+                }
+                if (count == 0) continue;
+                o -= count;
+                if (any != 0) f = fac[o];
+                found |= any != 0;
+            }
+            out[j] = found ? out[j] * f : out[j];
         }
     }
 }
 
+template <int R>
 __global__ __launch_bounds__(256) void k_burn(const float* __restrict__ zin,
                                               float* __restrict__ zout,
                                               const uint8_t* __restrict__ sf,
-                                              const int* __restrict__ off,
-                                              const float* __restrict__ fac, int n_off, int R,
-                                              int W, int H, float nodata_dem) {
-    float v[4];
-    int gx[4], gy[4];
-    burn_tile<false>(W, H, sf, off, fac, n_off, R, nodata_dem, zin, nullptr, v, gx, gy);
+                                              const float* __restrict__ fac, int n_off, int W, int H,
+                                              float nodata_dem) {
+    float v[BT_R];
+    int gx, gy;
+    burn_tile<false, R>(W, H, sf, fac, n_off, nodata_dem, zin, nullptr, v, gx, gy);
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-        if (gx[j] < W && gy[j] < H) zout[(size_t)gy[j] * W + gx[j]] = v[j];
+    for (int j = 0; j < BT_R; ++j)
+        if (gx < W && gy + j < H) zout[(size_t)(gy + j) * W + gx] = v[j];
 }
 
 // Quantisation of PitFillingAlgorithmCPUOpenMP.h:84-106 for one value.
@@ -320,25 +378,41 @@ __global__ __launch_bounds__(256) void k_quantize_minmax(float* __restrict__ z, 
 // driver: one pass over dem, error field and stream flags.  Each block
 // leaves its min/max partial in `part` (3 words per block) for
 // k_minmax_finish, so no block waits on the global words.
+template <int R>
 __global__ __launch_bounds__(256) void k_realistic_burn_quant(
     const float* __restrict__ dem, const float* __restrict__ e, const uint8_t* __restrict__ sf,
-    const int* __restrict__ off, const float* __restrict__ fac, int n_off, int R, int W, int H,
-    float nodata_dem, float* __restrict__ zq, uint32_t* __restrict__ part) {
-    float v[4];
-    int gx[4], gy[4];
-    burn_tile<true>(W, H, sf, off, fac, n_off, R, nodata_dem, dem, e, v, gx, gy);
+    const float* __restrict__ fac, int n_off, int W, int H, float nodata_dem, float* __restrict__ zq, uint32_t* __restrict__ part) {
+    float v[BT_R];
+    int gx, gy;
+    burn_tile<true, R>(W, H, sf, fac, n_off, nodata_dem, dem, e, v, gx, gy);
     uint32_t mn = 0xffffffffu, mx = 0u, bad = 0u;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        if (gx[j] < W && gy[j] < H) {
+    for (int j = 0; j < BT_R; ++j) {
+        if (gx < W && gy + j < H) {
             const float q = quantize_mm(v[j], nodata_dem, &bad);
-            zq[(size_t)gy[j] * W + gx[j]] = q;
+            zq[(size_t)(gy + j) * W + gx] = q;
             const uint32_t o = float_to_ordered(q);
             mn = min(mn, o);
             mx = max(mx, o);
         }
     }
     block_minmax_store(mn, mx, bad, part + 3 * ((size_t)blockIdx.y * gridDim.x + blockIdx.x));
+}
+
+// fn(a constant of the bevel radius): the radius is a template argument of
+// the burning kernels.
+template <class F>
+int with_radius(int R, F fn) {
+    static_assert(BH_MAX == 5, "every radius is listed");
+    switch (R) {
+        case 0: fn(std::integral_constant<int, 0>()); return CAGEO_OK;
+        case 1: fn(std::integral_constant<int, 1>()); return CAGEO_OK;
+        case 2: fn(std::integral_constant<int, 2>()); return CAGEO_OK;
+        case 3: fn(std::integral_constant<int, 3>()); return CAGEO_OK;
+        case 4: fn(std::integral_constant<int, 4>()); return CAGEO_OK;
+        case 5: fn(std::integral_constant<int, 5>()); return CAGEO_OK;
+        default: return CAGEO_ERR_ARG;
+    }
 }
 
 inline unsigned grid_1d(size_t n) {
@@ -366,19 +440,14 @@ int prepare_offsets(Context* c, int R) {
     l.sort([](const O& a, const O& b) {
         return a.d < b.d || (a.d == b.d && (a.y < b.y || (a.y == b.y && a.x < b.x)));
     });
-    std::vector<int> off;
     std::vector<float> fac;
     for (const O& o : l) {
-        off.push_back(o.x);
-        off.push_back(o.y);
         float xd = (float)(-o.x), yd = (float)(-o.y);
         float dist = std::sqrt(xd * xd + yd * yd);
         fac.push_back(dist / (float)R);
     }
     c->n_offsets = (int)fac.size();
     if (c->n_offsets > 0) {
-        CAGEO_HIP_TRY(hipMemcpyAsync(c->d_off, off.data(), off.size() * sizeof(int),
-                                     hipMemcpyHostToDevice, c->stream));
         CAGEO_HIP_TRY(hipMemcpyAsync(c->d_factor, fac.data(), fac.size() * sizeof(float),
                                      hipMemcpyHostToDevice, c->stream));
         CAGEO_HIP_TRY(hipStreamSynchronize(c->stream));
@@ -405,8 +474,10 @@ int launch_realistic(Context* c, const float* dem, float* field, float nodata) {
 int launch_burn(Context* c, const float* zin, float* zout, const uint8_t* sflags,
                 float nodata_dem) {
     dim3 grid((c->W + BT_X - 1) / BT_X, (c->H + BT_Y - 1) / BT_Y);
-    hipLaunchKernelGGL(k_burn, grid, dim3(256), 0, c->stream, zin, zout, sflags, c->d_off,
-                       c->d_factor, c->n_offsets, c->off_radius, c->W, c->H, nodata_dem);
+    CAGEO_TRY(with_radius(c->off_radius, [&](auto r) {
+        hipLaunchKernelGGL(k_burn<r.value>, grid, dim3(256), 0, c->stream, zin, zout, sflags,
+                           c->d_factor, c->n_offsets, c->W, c->H, nodata_dem);
+    }));
     CAGEO_HIP_TRY(hipGetLastError());
     return CAGEO_OK;
 }
@@ -427,9 +498,11 @@ size_t burn_blocks(int W, int H) {
 // well: they need no reset before it.
 int launch_realistic_burn_quant(Context* c, const float* dem, const float* e, float* zq) {
     dim3 grid((c->W + BT_X - 1) / BT_X, (c->H + BT_Y - 1) / BT_Y);
-    hipLaunchKernelGGL(k_realistic_burn_quant, grid, dim3(256), 0, c->stream, dem, e,
-                       c->d_sflags, c->d_off, c->d_factor, c->n_offsets, c->off_radius, c->W, c->H,
-                       c->nodata_dem, zq, c->d_bmm);
+    CAGEO_TRY(with_radius(c->off_radius, [&](auto r) {
+        hipLaunchKernelGGL(k_realistic_burn_quant<r.value>, grid, dim3(256), 0, c->stream, dem, e,
+                           c->d_sflags, c->d_factor, c->n_offsets, c->W, c->H, c->nodata_dem, zq,
+                           c->d_bmm);
+    }));
     hipLaunchKernelGGL(k_minmax_finish, dim3(1), dim3(MMF_T), 0, c->stream, c->d_bmm,
                        (int)burn_blocks(c->W, c->H), c->d_scal);
     CAGEO_HIP_TRY(hipGetLastError());
