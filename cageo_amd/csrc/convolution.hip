@@ -11,7 +11,7 @@
 //
 // Layout: output tiles of 64 x 64 cells staged through LDS with their
 // wrapped halo; taps are wave-uniform and come through scalar loads.
-#include "common.hpp"
+#include "tiles.hpp"
 
 namespace cageo {
 
@@ -22,7 +22,27 @@ __device__ inline int wrap_index(int i, int n) {
     return i < 0 ? i + n : i;
 }
 
-// Columns pass: out[y][x] = sum_fy in[wrap(y - r + fy)][x] * f[fy].
+// The same for the cells of a 64-cell tile and its halo of r on a raster of n
+// >= 64 + r cells, where an index is less than one period off.  The general
+// form is a division: with it, and with a division by the halo's width for
+// each cell of the rows pass, the passes spent more instructions on where to
+// load from than on the products (44 + 60 us at 4096^2, 39 + 45 now; 10 + 13
+// at 1000 x 777, 8 + 10 now).
+__device__ inline int wrap_tile(int i, int n, int r) {
+    if (n < TILE + r) return wrap_index(i, n);
+    return i < 0 ? i + n : i >= n ? i - n : i;
+}
+
+constexpr int TAPS = 16;  // taps of a step of the one-dimensional passes
+// Taps k0 .. k0 + TAPS - 1 (those below L), one a lane, to be read by
+// readlane: unlike a scalar load's, their wait leaves the LDS reads alone.
+__device__ inline float tap_step(const float* __restrict__ f, int k0, int L) {
+    return f[min(k0 + (int)(threadIdx.x & (TAPS - 1)), L - 1)];
+}
+
+// Columns pass: out[y][x] = sum_fy in[wrap(y - r + fy)][x] * f[fy].  A thread
+// has 16 outputs of a column and reads the 31 inputs of 16 taps at once (one
+// input slid in a tap, each read waited for, took twice as long).
 __global__ __launch_bounds__(256) void k_conv_cols(float* __restrict__ out,
                                                    const float* __restrict__ in,
                                                    const float* __restrict__ f, int r, int W,
@@ -30,19 +50,18 @@ __global__ __launch_bounds__(256) void k_conv_cols(float* __restrict__ out,
     extern __shared__ float lds[];  // (64 + 2r) rows x 64
     const int L = 2 * r + 1;
     const int x0 = blockIdx.x * TILE, y0 = blockIdx.y * TILE;
-    const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
+    const int tx = threadIdx.x & 63, ty = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int rows = TILE + 2 * r;
     const int x = x0 + tx;
+    const float* col = in + min(x, W - 1);  // (a column outside is not stored)
+    float taps = tap_step(f, 0, L);
     // batches of independent loads (each store waits only for its batch)
     constexpr int B = 8;
     for (int k0 = ty; k0 < rows; k0 += 4 * B) {
         float v[B];
 #pragma unroll
-        for (int j = 0; j < B; ++j) {
-            const int k = k0 + 4 * j;
-            v[j] = 0.0f;
-            if (k < rows && x < W) v[j] = in[(size_t)wrap_index(y0 - r + k, H) * W + x];
-        }
+        for (int j = 0; j < B; ++j)
+            v[j] = col[(size_t)wrap_tile(y0 - r + min(k0 + 4 * j, rows - 1), H, r) * W];
 #pragma unroll
         for (int j = 0; j < B; ++j)
             if (k0 + 4 * j < rows) lds[(k0 + 4 * j) * TILE + tx] = v[j];
@@ -51,13 +70,29 @@ __global__ __launch_bounds__(256) void k_conv_cols(float* __restrict__ out,
     float acc[STRIP];
 #pragma unroll
     for (int j = 0; j < STRIP; ++j) acc[j] = 0.0f;
-    const float* base = lds + (ty * STRIP) * TILE + tx;
-    for (int fy = 0; fy < L; ++fy) {
-        const float t = f[fy];
-        const float* p = base + fy * TILE;
+    const float* p = lds + (ty * STRIP) * TILE + tx;
+    int fy = 0;
+    for (; fy + TAPS <= L; fy += TAPS) {
+        const float next = tap_step(f, fy + TAPS, L);
+        float win[STRIP + TAPS - 1];
+#pragma unroll
+        for (int i = 0; i < STRIP + TAPS - 1; ++i) win[i] = p[(fy + i) * TILE];
+#pragma unroll
+        for (int u = 0; u < TAPS; ++u) {
+            const float t = lane_read(taps, u);
+#pragma unroll
+            for (int j = 0; j < STRIP; ++j) {
+                float prod = win[u + j] * t;
+                acc[j] = acc[j] + prod;
+            }
+        }
+        taps = next;
+    }
+    for (int u = 0; fy + u < L; ++u) {
+        const float t = lane_read(taps, u);
 #pragma unroll
         for (int j = 0; j < STRIP; ++j) {
-            float prod = p[j * TILE] * t;
+            float prod = p[(fy + u + j) * TILE] * t;
             acc[j] = acc[j] + prod;
         }
     }
@@ -74,45 +109,50 @@ __global__ __launch_bounds__(256) void k_conv_cols(float* __restrict__ out,
 // is transposed (blockIdx.x walks tile rows): blocks go round robin over the
 // 8 XCDs, so the left and right neighbours of a tile, whose halos overlap it,
 // are gridDim.x blocks away, on the same XCD and its L2 when gridDim.x is a
-// multiple of 8.
+// multiple of 8.  P: LDS cells a row (0: as many as the tile and its halo
+// have); a constant puts a thread's 16 rows into the reads' offsets.
+template <int P>
 __global__ __launch_bounds__(256) void k_conv_rows(float* __restrict__ out,
                                                    const float* __restrict__ in,
                                                    const float* __restrict__ f, int r, int W,
                                                    int H) {
-    extern __shared__ float lds[];  // 64 rows x (64 + 2r)
+    extern __shared__ float lds[];  // 64 rows x S, 64 + 2r cells of each used
     const int L = 2 * r + 1;
-    const int S = TILE + 2 * r;
+    const int cols = TILE + 2 * r, S = P ? P : cols;
     const int x0 = blockIdx.y * TILE, y0 = blockIdx.x * TILE;
-    const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-    constexpr int B = 8;  // batches of independent loads
-    for (int i0 = threadIdx.x; i0 < TILE * S; i0 += 256 * B) {
-        float v[B];
+    const int tx = threadIdx.x & 63, ty = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    float taps = tap_step(f, 0, L);
+    // A wave loads its strip's rows, 64 columns at a time, in batches of
+    // independent loads (a row or column outside is not stored).
+    for (int c0 = 0; c0 < cols; c0 += 64) {
+        const int c = c0 + tx;
+        const float* src = in + wrap_tile(x0 - r + min(c, cols - 1), W, r);
+        float v[STRIP];
 #pragma unroll
-        for (int j = 0; j < B; ++j) {
-            const int idx = i0 + 256 * j;
-            v[j] = 0.0f;
-            if (idx < TILE * S) {
-                const int row = idx / S, k = idx - row * S;
-                const int gy = y0 + row;
-                if (gy < H) v[j] = in[(size_t)gy * W + wrap_index(x0 - r + k, W)];
-            }
+        for (int j = 0; j < STRIP; ++j)
+            v[j] = src[(size_t)min(y0 + ty * STRIP + j, H - 1) * W];
+        if (c < cols) {
+#pragma unroll
+            for (int j = 0; j < STRIP; ++j) lds[(ty * STRIP + j) * S + c] = v[j];
         }
-#pragma unroll
-        for (int j = 0; j < B; ++j)
-            if (i0 + 256 * j < TILE * S) lds[i0 + 256 * j] = v[j];
     }
     __syncthreads();
     float acc[STRIP];
 #pragma unroll
     for (int j = 0; j < STRIP; ++j) acc[j] = 0.0f;
     const float* base = lds + (ty * STRIP) * S + tx;
-    for (int fx = 0; fx < L; ++fx) {
-        const float t = f[fx];
+    for (int k0 = 0; k0 < L; k0 += TAPS) {
+        const float next = tap_step(f, k0 + TAPS, L);
+        const int n = min(TAPS, L - k0);
+        for (int u = 0; u < n; ++u) {
+            const float t = lane_read(taps, u);
 #pragma unroll
-        for (int j = 0; j < STRIP; ++j) {
-            float prod = base[j * S + fx] * t;
-            acc[j] = acc[j] + prod;
+            for (int j = 0; j < STRIP; ++j) {
+                float prod = base[j * S + k0 + u] * t;
+                acc[j] = acc[j] + prod;
+            }
         }
+        taps = next;
     }
     const int x = x0 + tx;
     if (x < W) {
@@ -299,8 +339,16 @@ int launch_convolve_to(Context* c, float* field, float* buf, float** result) {
         hipLaunchKernelGGL(k_conv_cols, grid, dim3(256), lds, c->stream, buf, field,
                            c->d_filter, r, W, H);
         CAGEO_HIP_TRY(hipGetLastError());
-        hipLaunchKernelGGL(k_conv_rows, dim3(grid.y, grid.x), dim3(256), lds, c->stream, field, buf,
-                           c->d_filter, r, W, H);
+        const int cols = TILE + 2 * r;
+        auto rows = [&](auto kernel, int pitch) {
+            hipLaunchKernelGGL(kernel, dim3(grid.y, grid.x), dim3(256),
+                               (size_t)TILE * pitch * sizeof(float), c->stream, field, buf,
+                               c->d_filter, r, W, H);
+        };
+        if (cols <= 96) rows(k_conv_rows<96>, 96);
+        else if (cols <= 128) rows(k_conv_rows<128>, 128);
+        else if (cols <= 192) rows(k_conv_rows<192>, 192);
+        else rows(k_conv_rows<0>, cols);
         CAGEO_HIP_TRY(hipGetLastError());
         *result = field;
         return CAGEO_OK;
