@@ -525,7 +525,7 @@ class Context:
         _check(lib().cageo_to_byte_array(self._h, _ptr(out_bytes), _ptr(values)), "to_byte_array")
 
     def iteration_counts(self):
-        """(pit-fill rounds, pit-fill passes, flat passes, tracing rounds) of the last run."""
+        """(pit-fill lower bounds, pit-fill stages, flat passes, tracing jumps) of the last run."""
         out = np.zeros(4, np.int32)
         _check(lib().cageo_iteration_counts(self._h, out.ctypes.data), "iteration_counts")
         return tuple(int(v) for v in out)

@@ -456,9 +456,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
 // barrier a step.  Strides of 88 (x) and 72 (g) pixels put the 16 channels of
 // a fragment read in distinct bank groups.
 //
-// Bound by the loads' latency at two workgroups a CU.  The kernel it replaced
-// took one tap and 32 x 32 channels a workgroup and read every operand two
-// bytes at a time: 10.8 ms of the 17.3 ms of a step of 8 tiles of 512^2.
+// The kernel it replaced took one tap and 32 x 32 channels a workgroup and
+// read every operand two bytes at a time: 10.8 ms of the 17.3 ms of a step of
+// 8 tiles of 512^2.  This one takes 2.0 ms, some 0.3 PFLOP/s; how that divides
+// between the transposing stores to LDS, the loads and the matrix
+// instructions has not been measured.
 constexpr int WG_T = 512;        // threads
 constexpr int WG_XS = 88;        // pixels of a staged x channel: 8 (pixel -1 last), 64, 1, pad
 constexpr int WG_GS = 72;        // pixels of a staged g channel: 64, pad
@@ -766,8 +768,8 @@ __global__ __launch_bounds__(256) void k_relu_back_bias(const float* __restrict_
 // made it (act): g = bf16(act > 0 ? sum of dy's 2x2 block : 0), dy the first C
 // of Ctot channels at twice the size, and the sums of g as dbias partials.
 // One pass where k_upsample2_back and k_relu_back_bias took two, and the
-// tensor in between was stored: 0.27 ms of a 512^2 x 8 step's level 1 before,
-// 0.15 now.  A thread takes 8 channels; 8 * 256 is a multiple of C.
+// tensor in between was stored: 104 us a call over the three levels of a
+// 512^2 x 8 step, where the first of the two alone took 155.  A thread takes 8 channels; 8 * 256 is a multiple of C.
 __global__ __launch_bounds__(256) void k_up_relu_back(const float* __restrict__ dy,
                                                       const uint16_t* __restrict__ act,
                                                       uint16_t* __restrict__ g, int N, int H, int W,

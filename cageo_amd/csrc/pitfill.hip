@@ -36,12 +36,13 @@
 // Execution: one persistent launch without grid barriers.  Every 64 x 64
 // tile belongs to the workgroup that takes it in stage 0 (a workgroup takes
 // the next when done with one), which holds the tile it worked on last in LDS;
-// with as many workgroups as tiles none is ever loaded twice.  Tiles talk through an exchange buffer that holds each
-// tile's four border rows and columns: a workgroup that lowers a border cell
-// stores its side there and marks the rows this unsettles in the neighbour's
-// flag word, if any can change; the neighbour's owner finds the mark when it next polls, reloads
+// with as many workgroups as tiles none is ever loaded twice.  Tiles talk
+// through an exchange buffer that holds each tile's four border rows and
+// columns: a workgroup that lowers a border cell stores its side there and
+// marks the rows this unsettles in the neighbour's flag word, if any can
+// change; the neighbour's owner finds the mark when it next polls, reloads
 // the ring and solves those rows.  A stage is over when no flag is up and no
-// tile is at work (see pf_publish).  
+// tile is at work (see pf_publish).
 //
 // What bounds it: at 4096^2 the row steps' issue (four waves a SIMD), below
 // 1024 tiles the chain of dependent visits (a visit's solve plus some 5 us

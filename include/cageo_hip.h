@@ -274,8 +274,9 @@ int cageo_batch_configure_tile(cageo_batch* batch, int tile, int persistent_work
                                int conv_rows);
 
 /* Iteration counts of the last fixed-point launches on this context: pit
- * fill rounds, pit fill passes, flat-resolution passes, tracing exit-jump
- * rounds (the reference's PitFillingAlgorithm::iter-style counters).
+ * fill lower bounds, pit fill stages (both bounds), flat-resolution passes,
+ * most exit jumps of a tracing chain (the reference's
+ * PitFillingAlgorithm::iter-style counters).
  * `out` holds 4 ints. */
 int cageo_iteration_counts(cageo_context* ctx, int32_t* out);
 /* Launch settings of this context: persistent_workgroups for the persistent
