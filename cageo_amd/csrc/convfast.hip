@@ -17,16 +17,11 @@
 // outputs (4 columns as a float4); for every term the plane's tile with its
 // wrapped column halo is staged in LDS and read as float4 pairs (8 values
 // for 4 taps x 4 outputs), accumulating all terms in registers.
-#include "common.hpp"
+#include "tiles.hpp"
 
 namespace cageo {
 
 namespace {
-
-__device__ inline int wrap_i(int i, int n) {
-    i %= n;
-    return i < 0 ? i + n : i;
-}
 
 constexpr int LR_KG = 4;  // terms per column-pass launch slice
 
@@ -40,17 +35,18 @@ __global__ __launch_bounds__(256) void k_lr_cols(float* __restrict__ planes,
     extern __shared__ float lds[];  // (64 + LC) rows x 64; rows from 64 + 2r on are zero
     const int x0 = blockIdx.x * TILE, y0 = blockIdx.y * TILE;
     const int k0 = blockIdx.z * LR_KG;
-    const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
+    const int tx = threadIdx.x & 63, ty = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int rows = TILE + 2 * r, lrows = TILE + LC;
     const int x = x0 + tx;
+    const float* col = in + min(x, W - 1);  // (a column outside is not stored)
     constexpr int B = 8;  // batches of independent loads
     for (int k0 = ty; k0 < lrows; k0 += 4 * B) {
         float v[B];
 #pragma unroll
         for (int j = 0; j < B; ++j) {
             const int k = k0 + 4 * j;
-            v[j] = 0.0f;
-            if (k < rows && x < W) v[j] = in[(size_t)wrap_i(y0 - r + k, H) * W + x];
+            v[j] = col[(size_t)wrap_tile(y0 - r + min(k, rows - 1), H, r) * W];
+            if (k >= rows) v[j] = 0.0f;
         }
 #pragma unroll
         for (int j = 0; j < B; ++j)
@@ -164,22 +160,24 @@ __global__ __launch_bounds__(256) void k_lr_rows(float* __restrict__ out,
     const size_t n = (size_t)W * H;
     for (int k = 0; k < K; ++k) {
         const float* P = planes + (size_t)k * n;
-        constexpr int B = 8;  // batches of independent loads
-        for (int i0 = threadIdx.x; i0 < TILE * S; i0 += 256 * B) {
-            float v[B];
+        // A wave loads 16 rows, 64 columns at a time, in one batch (a row
+        // outside is not stored; the columns past the halo, whose taps are
+        // zero, hold zeros).  A division a cell for its row, and one for its
+        // wrap, took more instructions than the products: 570 us
+        // at 3000 x 2301 (exponential, 200 m), 340 now.
+        const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        for (int c0 = 0; c0 < S; c0 += 64) {
+            const int cc = c0 + lane;
+            const float* src = P + wrap_tile(x0 - r + min(cc, cols - 1), W, r);
+            float v[STRIP];
 #pragma unroll
-            for (int j = 0; j < B; ++j) {
-                const int idx = i0 + 256 * j;
-                v[j] = 0.0f;
-                if (idx < TILE * S) {
-                    const int row = idx / S, cc = idx - row * S;
-                    const int gy = y0 + row;
-                    if (cc < cols && gy < H) v[j] = P[(size_t)gy * W + wrap_i(x0 - r + cc, W)];
-                }
+            for (int j = 0; j < STRIP; ++j)
+                v[j] = src[(size_t)min(y0 + wave * STRIP + j, H - 1) * W];
+            if (cc < S) {
+#pragma unroll
+                for (int j = 0; j < STRIP; ++j)
+                    lds[(wave * STRIP + j) * S + cc] = cc < cols ? v[j] : 0.0f;
             }
-#pragma unroll
-            for (int j = 0; j < B; ++j)
-                if (i0 + 256 * j < TILE * S) lds[i0 + 256 * j] = v[j];
         }
         __syncthreads();
         // rows ty4 + 16 a; each step takes one tap quadruple for all four

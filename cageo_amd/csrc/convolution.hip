@@ -17,22 +17,6 @@ namespace cageo {
 
 namespace {
 
-__device__ inline int wrap_index(int i, int n) {
-    i %= n;
-    return i < 0 ? i + n : i;
-}
-
-// The same for the cells of a 64-cell tile and its halo of r on a raster of n
-// >= 64 + r cells, where an index is less than one period off.  The general
-// form is a division: with it, and with a division by the halo's width for
-// each cell of the rows pass, the passes spent more instructions on where to
-// load from than on the products (44 + 60 us at 4096^2, 39 + 45 now; 10 + 13
-// at 1000 x 777, 8 + 10 now).
-__device__ inline int wrap_tile(int i, int n, int r) {
-    if (n < TILE + r) return wrap_index(i, n);
-    return i < 0 ? i + n : i >= n ? i - n : i;
-}
-
 constexpr int TAPS = 16;  // taps of a step of the one-dimensional passes
 // Taps k0 .. k0 + TAPS - 1 (those below L), one a lane, to be read by
 // readlane: unlike a scalar load's, their wait leaves the LDS reads alone.
