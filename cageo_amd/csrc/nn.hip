@@ -17,6 +17,8 @@
 // MFMA operand layout (16x16x32, wave64): lane l holds 8 consecutive K values
 // of row (l % 16) of A and of column (l % 16) of B, K block (l / 16); the
 // accumulator holds rows 4*(l / 16) + r, r = 0..3, of column l % 16.
+#include <type_traits>
+
 #include "common.hpp"
 
 namespace cageo {
@@ -131,26 +133,16 @@ __global__ __launch_bounds__(256) void k_conv3x3(ConvIn ci, const uint16_t* __re
     }
 }
 
-// The same convolution with its operands staged in LDS, for any W and H (the
-// tiles at the right and lower edges load zeros and store what lies inside).
-// A workgroup computes a tile of 4 RW rows x 64 pixels
-// (wave w: rows w RW .. w RW + RW - 1, 4 accumulator tiles of 16 pixels
-// each) x 16*NT output channels; with RW = 2 each weight fragment read
-// feeds twice the MFMAs (the 32-channel layers).  Per 32-channel slice of
-// the input it stages the (4 RW + 2) x 66 input pixels the 9 taps read (zero outside the image, upsampling and concatenation folded
-// into the loads) and the slice's weights of all 9 taps, then runs the 9
-// taps from LDS: each staged value is read from memory once per
-// workgroup instead of once per tap and wave.  Pixel rows in LDS are
-// padded to 40 bf16 (80 bytes) so 16 lanes reading 16 consecutive pixels
-// hit 16 distinct 4-bank groups.
-//
-// Without an fp32 output the results go out through LDS: the workgroup's
-// bias + ReLU outputs, rounded to bf16, are staged there, then written
-// with 16-byte stores (a pixel's channels are contiguous), and the fused
-// consumers of the output read them there (ConvFuse): the 2x2 average pool
-// and the 1x1 head, each in the same arithmetic as its own kernel
-// (k_avgpool2, k_head), so a fused layer gives the same bits as the layer
-// followed by that kernel.
+// The same convolution with its operands staged in LDS: for W % 64 == 0 and
+// H % 4 == 0, and for any W and H where the input has one slice of 32 channels
+// (EDGE: the tiles at the right and lower edges load zeros and store what
+// lies inside).  A workgroup computes a tile of 4 rows x 64 pixels (a wave a
+// row, 4 accumulator tiles of 16 pixels) x 16*NT output channels.  Per
+// 32-channel slice of the input it stages the 6 x 66 input pixels the 9 taps
+// read (zero outside the image, upsampling and concatenation folded into the
+// loads) and the slice's weights of all 9 taps, then runs the 9 taps from LDS:
+// each staged value is read from memory once per workgroup instead of once
+// per tap and wave.
 constexpr int CL_TX = 64;
 
 // Place (in bf16) of 16-byte chunk c (0..3) of staged row r of the LDS
@@ -193,10 +185,12 @@ __device__ inline void add8(float (&s)[8], uint4 v) {
         s[2 * k + 1] += bf2f((uint16_t)(u[k] >> 16));
     }
 }
-// Sums over the workgroup (256 threads) of each thread's 8 channels
+// Sums over the workgroup (WAVES waves) of each thread's 8 channels
 // 8 (threadIdx.x % CH) .. + 7, CH a power of two up to 32, added to this
 // workgroup's slot of the partial sums: atomics of thousands of workgroups on
-// one row of words would queue (23 ns each).  `part`: 4 x 8 CH floats of LDS.
+// one row of words would queue (23 ns each).  `part`: WAVES x 8 CH floats of
+// LDS.
+template <int WAVES = 4>
 __device__ inline void bias_partials(float (&s)[8], int CH, float* part, float* dbias, int cout,
                                      int co0) {
     for (int off = 32; off >= CH; off >>= 1)
@@ -207,27 +201,164 @@ __device__ inline void bias_partials(float (&s)[8], int CH, float* part, float* 
 #pragma unroll
         for (int k = 0; k < 8; ++k) part[wave * C + 8 * lane + k] = s[k];
     __syncthreads();
-    if ((int)threadIdx.x < C)
-        atomicAdd(&dbias[(size_t)(blockIdx.x % BIAS_SLOTS) * cout + co0 + threadIdx.x],
-                  (part[threadIdx.x] + part[C + threadIdx.x]) +
-                      (part[2 * C + threadIdx.x] + part[3 * C + threadIdx.x]));
+    if ((int)threadIdx.x < C) {
+        float v = part[threadIdx.x];
+        for (int k = 1; k < WAVES; ++k) v += part[k * C + threadIdx.x];
+        atomicAdd(&dbias[(size_t)(blockIdx.x % BIAS_SLOTS) * cout + co0 + threadIdx.x], v);
+    }
+}
+
+// What a workgroup of ROWS x CW waves makes of its accumulators: wave k's are
+// row k % ROWS of the tile of ROWS rows x 64 pixels and output channels
+// 16 NT (k / ROWS) on.  `smem` holds conv_out_words words that no wave uses
+// any more.
+//
+// Without an fp32 output the results go out through LDS: the workgroup's
+// bias + ReLU outputs, rounded to bf16, are staged there, then written
+// with 16-byte stores (a pixel's channels are contiguous), and the fused
+// consumers of the output read them there (ConvFuse): the 2x2 average pool
+// and the 1x1 head, each in the same arithmetic as its own kernel
+// (k_avgpool2, k_head), so a fused layer gives the same bits as the layer
+// followed by that kernel.
+template <int NT, int ROWS, int CW>
+constexpr int conv_out_words() {
+    constexpr int CO = 16 * NT * CW, NPX = ROWS * CL_TX;
+    return NPX * (CO + 8) > CO * (NPX + 2) ? NPX * (CO + 8) : CO * (NPX + 2);
+}
+template <int NT, int ROWS, int CW, bool EDGE>
+__device__ __forceinline__ void conv_out(f32x4 (&acc)[4][NT], uint16_t* smem,
+                                         const float* __restrict__ bias, uint16_t* __restrict__ out,
+                                         float* __restrict__ outf, const ConvFuse& fz, int n, int y0,
+                                         int x0, int co0, int H, int W, int Cout, int relu) {
+    constexpr int T = 64 * ROWS * CW, CO = 16 * NT * CW;
+    constexpr int NPX = ROWS * CL_TX;    // pixels of the output tile
+    constexpr int PS = CO + 8;           // staged pixel stride (bf16), padded by 16 bytes
+    constexpr int HP = NPX + 2;          // staged channel stride of the head's layout
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int row = lane & 15, kb = lane >> 4;
+    const int wr = wave % ROWS, wc = 16 * NT * (wave / ROWS);
+    if (outf) {  // fp32 output too: straight from the accumulators
+        const long long prow = ((long long)n * H + y0 + wr) * W + x0;
+        const int wx = W - x0;  // the tile's pixels inside
+        if (EDGE && y0 + wr >= H) return;
+#pragma unroll
+        for (int q = 0; q < NT; ++q) {
+            const int co = co0 + wc + 16 * q + row;  // accumulator column = lane % 16
+            const float bias_co = bias ? bias[co] : 0.0f;
+#pragma unroll
+            for (int m = 0; m < 4; ++m)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    if (EDGE && 16 * m + 4 * kb + r >= wx) continue;
+                    const long long pp = prow + 16 * m + 4 * kb + r;
+                    float v = acc[m][q][r] + bias_co;
+                    if (relu) v = fmaxf(v, 0.0f);
+                    if (out) out[pp * Cout + co] = f2bf(v);
+                    outf[pp * Cout + co] = v;
+                }
+        }
+        return;
+    }
+    // the output tile's pixel (0, 0) in the NHWC raster; the head layout is
+    // channel-major (a thread then reads its pixel's channels in order, lanes
+    // on consecutive pixels), the other pixel-major
+    const size_t pix0 = ((size_t)n * H + y0) * W + x0;
+    const bool head = fz.prob != nullptr;
+#pragma unroll
+    for (int q = 0; q < NT; ++q) {
+        const int c = wc + 16 * q + row;  // accumulator column = lane % 16
+        const float bias_co = bias ? bias[co0 + c] : 0.0f;
+#pragma unroll
+        for (int m = 0; m < 4; ++m)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int px = wr * CL_TX + 16 * m + 4 * kb + r;
+                float v = acc[m][q][r] + bias_co;
+                if (relu) v = fmaxf(v, 0.0f);
+                smem[head ? c * HP + px : px * PS + c] = f2bf(v);
+            }
+    }
+    __syncthreads();
+    if (head) {  // CO == Cout (the host checks): the workgroup holds every channel
+        for (int px = threadIdx.x; px < NPX; px += T) {
+            if (EDGE && (px / CL_TX >= H - y0 || px % CL_TX >= W - x0)) continue;
+            float s = fz.head_b[0];
+            for (int c = 0; c < CO; ++c) s += fz.head_w[c] * bf2f(smem[c * HP + px]);
+            fz.prob[pix0 + (size_t)(px / CL_TX) * W + px % CL_TX] =
+                fz.sigmoid ? 1.0f / (1.0f + expf(-s)) : s;
+        }
+        return;
+    }
+    constexpr int CH = CO / 8;  // 16-byte chunks of a pixel's channels
+    if (fz.mask) {
+        float sum[8] = {};
+#pragma unroll
+        for (int i0 = 0; i0 < NPX * CH; i0 += T) {
+            const int i = i0 + threadIdx.x, px = i / CH, part = i - px * CH;
+            if (EDGE && (px / CL_TX >= H - y0 || px % CL_TX >= W - x0)) continue;
+            const size_t o = (pix0 + (size_t)(px / CL_TX) * W + px % CL_TX) * Cout + co0 + 8 * part;
+            const uint4 v = relu_mask(*reinterpret_cast<const uint4*>(smem + px * PS + 8 * part),
+                                      *reinterpret_cast<const uint4*>(fz.mask + o));
+            *reinterpret_cast<uint4*>(out + o) = v;
+            add8(sum, v);
+        }
+        __syncthreads();  // the staged outputs are read
+        bias_partials<ROWS * CW>(sum, CH, reinterpret_cast<float*>(smem), fz.dbias, Cout, co0);
+        return;
+    }
+    if (out) {
+        for (int i = threadIdx.x; i < NPX * CH; i += T) {
+            const int px = i / CH, part = i - px * CH;
+            if (EDGE && (px / CL_TX >= H - y0 || px % CL_TX >= W - x0)) continue;
+            const size_t g = (pix0 + (size_t)(px / CL_TX) * W + px % CL_TX) * Cout + co0 + 8 * part;
+            *reinterpret_cast<uint4*>(out + g) =
+                *reinterpret_cast<const uint4*>(smem + px * PS + 8 * part);
+        }
+    }
+    if (ROWS > 1 && fz.pool) {
+        const int Wo = W / 2;
+        const size_t q0 = ((size_t)n * (H / 2) + y0 / 2) * Wo + x0 / 2;
+        for (int i = threadIdx.x; i < NPX / 4 * CH; i += T) {
+            const int pp = i / CH, part = i - pp * CH;
+            const int py = pp / (CL_TX / 2), px = pp - py * (CL_TX / 2);
+            if (EDGE && (2 * py >= H - y0 || 2 * px >= W - x0)) continue;
+            const uint16_t* s00 = smem + (2 * py * CL_TX + 2 * px) * PS + 8 * part;
+            const uint4 a = *reinterpret_cast<const uint4*>(s00);                 // (2y, 2x)
+            const uint4 b = *reinterpret_cast<const uint4*>(s00 + PS);            // (2y, 2x+1)
+            const uint4 c = *reinterpret_cast<const uint4*>(s00 + CL_TX * PS);    // (2y+1, 2x)
+            const uint4 d = *reinterpret_cast<const uint4*>(s00 + (CL_TX + 1) * PS);
+            const uint32_t ua[4] = {a.x, a.y, a.z, a.w}, ub[4] = {b.x, b.y, b.z, b.w};
+            const uint32_t uc[4] = {c.x, c.y, c.z, c.w}, ud[4] = {d.x, d.y, d.z, d.w};
+            uint32_t res[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                uint32_t h2 = 0;
+#pragma unroll
+                for (int hh = 0; hh < 2; ++hh) {
+                    const int sh = 16 * hh;
+                    const float sum = bf2f((uint16_t)(ua[k] >> sh)) + bf2f((uint16_t)(ub[k] >> sh)) +
+                                      bf2f((uint16_t)(uc[k] >> sh)) + bf2f((uint16_t)(ud[k] >> sh));
+                    h2 |= (uint32_t)f2bf(0.25f * sum) << sh;
+                }
+                res[k] = h2;
+            }
+            *reinterpret_cast<uint4*>(fz.pool + (q0 + (size_t)py * Wo + px) * Cout + co0 + 8 * part) =
+                make_uint4(res[0], res[1], res[2], res[3]);
+        }
+    }
 }
 
 // EDGE: W or H is no multiple of the tile's (else the stores need no tests:
 // with them a 4096^2 prediction takes 2 % longer).
-template <int NT, int RW, int WPE, bool EDGE>
+template <int NT, int WPE, bool EDGE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void k_conv3x3_lds(ConvIn ci, const uint16_t* __restrict__ w,
                                                      const float* __restrict__ bias,
                                                      uint16_t* __restrict__ out,
                                                      float* __restrict__ outf, ConvFuse fz,
                                                      int N, int H, int W, int Cout, int relu) {
-    constexpr int TY = 4 * RW, AX = CL_TX + 2, AY = TY + 2, CO = 16 * NT;
-    constexpr int TAP_UNROLL = RW == 1 ? 9 : 1;  // two rows a wave: registers run short
+    constexpr int TY = 4, AX = CL_TX + 2, AY = TY + 2, CO = 16 * NT;
     constexpr int SA_N = AY * AX * 32, SB_N = 9 * CO * 32;
-    constexpr int NPX = TY * CL_TX;      // pixels of the output tile
-    constexpr int PS = CO + 8;           // staged pixel stride (bf16), padded by 16 bytes
-    constexpr int HP = NPX + 2;          // staged channel stride of the head's layout
-    static_assert(NPX * PS <= SA_N + SB_N && CO * HP <= SA_N + SB_N, "epilogue staging");
+    static_assert(conv_out_words<NT, 4, 1>() <= SA_N + SB_N, "epilogue staging");
     __shared__ __align__(16) uint16_t smem[SA_N + SB_N];
     uint16_t* const sa = smem;
     uint16_t* const sb = smem + SA_N;
@@ -241,9 +372,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
     const int x0 = tx * CL_TX, y0 = ty * TY;
     const int co0 = blockIdx.y * CO;
     const int Cin = ci.C1 + ci.C2;
-    f32x4 acc[4 * RW][NT];
+    f32x4 acc[4][NT];
 #pragma unroll
-    for (int m = 0; m < 4 * RW; ++m)
+    for (int m = 0; m < 4; ++m)
 #pragma unroll
         for (int q = 0; q < NT; ++q) acc[m][q] = f32x4{0.f, 0.f, 0.f, 0.f};
     // Slice c's loads are issued before slice c - 32's MFMAs and stored to
@@ -303,134 +434,205 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
         }
         __syncthreads();
         if (c + 32 < Cin) load_slice(c + 32);
-#pragma unroll TAP_UNROLL
+#pragma unroll
         for (int tap = 0; tap < 9; ++tap) {
             const int dy = tap / 3, dx = tap % 3;  // halo-shifted offsets 0..2
-            bf16x8 a[4 * RW], b[NT];
+            bf16x8 a[4], b[NT];
 #pragma unroll
-            for (int m = 0; m < 4 * RW; ++m)
+            for (int m = 0; m < 4; ++m)
                 a[m] = as_bf16x8(*reinterpret_cast<const uint4*>(
-                    &sa[cl_at((wave * RW + m / 4 + dy) * AX + 16 * (m % 4) + row + dx, kb)]));
+                    &sa[cl_at((wave + dy) * AX + 16 * m + row + dx, kb)]));
 #pragma unroll
             for (int q = 0; q < NT; ++q)
                 b[q] = as_bf16x8(*reinterpret_cast<const uint4*>(
                     &sb[cl_at(tap * CO + 16 * q + row, kb)]));
 #pragma unroll
-            for (int m = 0; m < 4 * RW; ++m)
+            for (int m = 0; m < 4; ++m)
 #pragma unroll
                 for (int q = 0; q < NT; ++q)
                     acc[m][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m], b[q], acc[m][q], 0, 0, 0);
         }
     }
-    if (outf) {  // fp32 output too: straight from the accumulators
-        const long long prow = ((long long)n * H + y0 + wave * RW) * W + x0;
-        const int wy = H - y0 - wave * RW, wx = W - x0;  // the tile's rows and pixels inside
-#pragma unroll
-        for (int q = 0; q < NT; ++q) {
-            const int co = co0 + 16 * q + row;  // accumulator column = lane % 16
-            const float bias_co = bias ? bias[co] : 0.0f;
-#pragma unroll
-            for (int m = 0; m < 4 * RW; ++m)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    if (EDGE && (m / 4 >= wy || 16 * (m % 4) + 4 * kb + r >= wx)) continue;
-                    const long long pp = prow + (long long)(m / 4) * W + 16 * (m % 4) + 4 * kb + r;
-                    float v = acc[m][q][r] + bias_co;
-                    if (relu) v = fmaxf(v, 0.0f);
-                    if (out) out[pp * Cout + co] = f2bf(v);
-                    outf[pp * Cout + co] = v;
-                }
-        }
-        return;
-    }
     __syncthreads();  // every wave's operand reads of the last slice are done
-    // the output tile's pixel (0, 0) in the NHWC raster; the head layout is
-    // channel-major (a thread then reads its pixel's channels in order, lanes
-    // on consecutive pixels), the other pixel-major
-    const size_t pix0 = ((size_t)n * H + y0) * W + x0;
-    const bool head = fz.prob != nullptr;
+    conv_out<NT, 4, 1, EDGE>(acc, smem, bias, out, outf, fz, n, y0, x0, co0, H, W, Cout, relu);
+}
+
+// The convolution for any W and H with its sums in k_conv3x3's order, all
+// channels of tap 0 first, then those of tap 1, and so on (k_conv3x3_lds goes
+// slice by slice), so that an image's outputs have the same bits whichever of
+// the two kernels its size goes to.  The order needs every channel of the
+// pixels at hand: a workgroup stages all of them once, in slices of 32 (see
+// cl_at), an upsampled input at its own resolution, and then runs the steps,
+// a slice of a tap each, with a step's weights through LDS.  While step j's
+// products run, step j + 1's operands come from LDS, the weights of j + 2 go
+// there and those of the three after it are on their way from memory.
+// ROWS rows x 64 pixels a workgroup, ROWS x CW waves, each a row and 16 NT
+// output channels.
+// Bound by the LDS reads of a step and the barrier that ends it (384 cycles of
+// reads for 256 of products with eight waves); the pixels take the LDS of one
+// such workgroup a CU, so eight waves are better than four that reuse more
+// (384 -> 128 channels upsampled at 252 x 176: 82 us against 101), and staging
+// an upsampled input at full size took 120.  A 1001 x 700 prediction takes
+// 0.52 ms; with k_conv3x3 in its place 1.18, with the staged kernel's order
+// 0.44.
+constexpr int CT_LDS = 160 * 1024;
+// Staged pixels of an input: whole eights, so that cl_at of a slice's pixel is
+// the slice's place plus the pixel's.
+constexpr int CT_AX = CL_TX + 2, CT_HX = CL_TX / 2 + 2;  // a row of them; of an upsampled input's
+constexpr int conv_taps_px(int rows, int up) {
+    return (up ? (rows / 2 + 2) * CT_HX + 7 : (rows + 2) * CT_AX + 7) & ~7;
+}
+// Words of LDS: the pixels, 8 that are written for none, two steps' weights.
+constexpr int conv_taps_words(int rows, int block, int c1, int up1, int c2) {
+    return conv_taps_px(rows, up1) * c1 + conv_taps_px(rows, 0) * c2 + 8 + 2 * 32 * block;
+}
+template <int NT, int ROWS, int CW>
+__global__ __launch_bounds__(64 * ROWS * CW) __attribute__((amdgpu_waves_per_eu(2, 4))) void k_conv3x3_taps(
+    ConvIn ci, const uint16_t* __restrict__ w, const float* __restrict__ bias,
+    uint16_t* __restrict__ out, float* __restrict__ outf, ConvFuse fz, int N, int H, int W, int Cout,
+    int relu) {
+    extern __shared__ __align__(16) uint16_t staged[];  // [slices][pixels][32], weights [2][CO][32]
+    constexpr int T = 64 * ROWS * CW, CO = 16 * NT * CW;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int row = lane & 15, kb = lane >> 4;
+    const int tiles_x = (W + CL_TX - 1) / CL_TX, tiles_y = (H + ROWS - 1) / ROWS;
+    const int t = blockIdx.x;
+    const int n = t / (tiles_x * tiles_y);
+    const int y0 = (t / tiles_x) % tiles_y * ROWS, x0 = t % tiles_x * CL_TX;
+    const int co0 = blockIdx.y * CO;
+    const int Cin = ci.C1 + ci.C2;
+    const int np1 = conv_taps_px(ROWS, ci.up1), np2 = conv_taps_px(ROWS, 0);
+    const int words = np1 * ci.C1 + np2 * ci.C2;
+    // Pixels of an input of Hs x Ws from (ys, xs) on, AX a row, to staged
+    // pixel `r0` on: 16 bytes a load, a pixel's channels and then the next
+    // pixel's by consecutive threads, B loads a thread under way (a pixel
+    // outside loads the first one).
+    auto stage = [&](auto row_of, const uint16_t* src, int C, int np, int Hs, int Ws, int ys, int xs,
+                     int r0) __attribute__((always_inline)) {
+        constexpr int B = 8, AX = row_of.value;
+        const int cq = C / 8, dp = T / cq, dq = T - dp * cq;
+        int p = threadIdx.x / cq, q = threadIdx.x - p * cq;
+        while (__any(p < np)) {
+            bf16x8 v[B];
+            int at[B];
+            uint32_t in = 0;
 #pragma unroll
-    for (int q = 0; q < NT; ++q) {
-        const int c = 16 * q + row;  // accumulator column = lane % 16
-        const float bias_co = bias ? bias[co0 + c] : 0.0f;
-#pragma unroll
-        for (int m = 0; m < 4 * RW; ++m)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int px = (wave * RW + m / 4) * CL_TX + 16 * (m % 4) + 4 * kb + r;
-                float v = acc[m][q][r] + bias_co;
-                if (relu) v = fmaxf(v, 0.0f);
-                smem[head ? c * HP + px : px * PS + c] = f2bf(v);
-            }
-    }
-    __syncthreads();
-    if (head) {  // CO == Cout (the host checks): the workgroup holds every channel
-        for (int px = threadIdx.x; px < NPX; px += 256) {
-            if (EDGE && (px / CL_TX >= H - y0 || px % CL_TX >= W - x0)) continue;
-            float s = fz.head_b[0];
-            for (int c = 0; c < CO; ++c) s += fz.head_w[c] * bf2f(smem[c * HP + px]);
-            fz.prob[pix0 + (size_t)(px / CL_TX) * W + px % CL_TX] =
-                fz.sigmoid ? 1.0f / (1.0f + expf(-s)) : s;
-        }
-        return;
-    }
-    constexpr int CH = CO / 8;  // 16-byte chunks of a pixel's channels
-    if (fz.mask) {
-        float sum[8] = {};
-#pragma unroll
-        for (int i0 = 0; i0 < NPX * CH; i0 += 256) {
-            const int i = i0 + threadIdx.x, px = i / CH, part = i - px * CH;
-            if (EDGE && (px / CL_TX >= H - y0 || px % CL_TX >= W - x0)) continue;
-            const size_t o = (pix0 + (size_t)(px / CL_TX) * W + px % CL_TX) * Cout + co0 + 8 * part;
-            const uint4 v = relu_mask(*reinterpret_cast<const uint4*>(smem + px * PS + 8 * part),
-                                      *reinterpret_cast<const uint4*>(fz.mask + o));
-            *reinterpret_cast<uint4*>(out + o) = v;
-            add8(sum, v);
-        }
-        __syncthreads();  // the staged outputs are read
-        bias_partials(sum, CH, reinterpret_cast<float*>(smem), fz.dbias, Cout, co0);
-        return;
-    }
-    if (out) {
-        for (int i = threadIdx.x; i < NPX * CH; i += 256) {
-            const int px = i / CH, part = i - px * CH;
-            if (EDGE && (px / CL_TX >= H - y0 || px % CL_TX >= W - x0)) continue;
-            const size_t g = (pix0 + (size_t)(px / CL_TX) * W + px % CL_TX) * Cout + co0 + 8 * part;
-            *reinterpret_cast<uint4*>(out + g) =
-                *reinterpret_cast<const uint4*>(smem + px * PS + 8 * part);
-        }
-    }
-    if (fz.pool) {
-        const int Wo = W / 2;
-        const size_t q0 = ((size_t)n * (H / 2) + y0 / 2) * Wo + x0 / 2;
-        for (int i = threadIdx.x; i < NPX / 4 * CH; i += 256) {
-            const int pp = i / CH, part = i - pp * CH;
-            const int py = pp / (CL_TX / 2), px = pp - py * (CL_TX / 2);
-            if (EDGE && (2 * py >= H - y0 || 2 * px >= W - x0)) continue;
-            const uint16_t* s00 = smem + (2 * py * CL_TX + 2 * px) * PS + 8 * part;
-            const uint4 a = *reinterpret_cast<const uint4*>(s00);                 // (2y, 2x)
-            const uint4 b = *reinterpret_cast<const uint4*>(s00 + PS);            // (2y, 2x+1)
-            const uint4 c = *reinterpret_cast<const uint4*>(s00 + CL_TX * PS);    // (2y+1, 2x)
-            const uint4 d = *reinterpret_cast<const uint4*>(s00 + (CL_TX + 1) * PS);
-            const uint32_t ua[4] = {a.x, a.y, a.z, a.w}, ub[4] = {b.x, b.y, b.z, b.w};
-            const uint32_t uc[4] = {c.x, c.y, c.z, c.w}, ud[4] = {d.x, d.y, d.z, d.w};
-            uint32_t res[4];
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                uint32_t h2 = 0;
-#pragma unroll
-                for (int hh = 0; hh < 2; ++hh) {
-                    const int sh = 16 * hh;
-                    const float sum = bf2f((uint16_t)(ua[k] >> sh)) + bf2f((uint16_t)(ub[k] >> sh)) +
-                                      bf2f((uint16_t)(uc[k] >> sh)) + bf2f((uint16_t)(ud[k] >> sh));
-                    h2 |= (uint32_t)f2bf(0.25f * sum) << sh;
+            for (int k = 0; k < B; ++k) {
+                const int py = p / AX, yy = ys + py, xx = xs + p - py * AX;
+                const bool inside = p < np && yy >= 0 && xx >= 0 && yy < Hs && xx < Ws;
+                const size_t o = (((size_t)n * Hs + yy) * Ws + xx) * C + 8 * q;
+                v[k] = *reinterpret_cast<const bf16x8*>(src + (inside ? o : 0));
+                in |= inside ? 1u << k : 0u;
+                at[k] = p < np ? cl_at(r0 + (q >> 2) * np + p, q & 3) : words;
+                p += dp;
+                q += dq;
+                if (q >= cq) {
+                    q -= cq;
+                    ++p;
                 }
-                res[k] = h2;
             }
-            *reinterpret_cast<uint4*>(fz.pool + (q0 + (size_t)py * Wo + px) * Cout + co0 + 8 * part) =
-                make_uint4(res[0], res[1], res[2], res[3]);
+#pragma unroll
+            for (int k = 0; k < B; ++k)
+                *reinterpret_cast<bf16x8*>(&staged[at[k]]) = (in >> k) & 1u ? v[k] : bf16x8{};
+        }
+    };
+    constexpr int D = 3;        // steps a round: 9 taps make whole rounds of them
+    constexpr int WT = CO * 4;  // threads with weights to stage
+    static_assert(WT <= T, "a load a thread");
+    bf16x8 a[D][4], b[D][NT], wv[D];
+    // Weights: of the step to load (past the last, step 0's), this thread's
+    // place in them, and where they go.
+    const int wt = min((int)threadIdx.x, WT - 1);
+    const uint32_t wlane = (uint32_t)((co0 + (wt >> 2)) * Cin + 8 * (wt & 3));
+    const int wput = words + 8 + cl_at(wt >> 2, wt & 3);
+    int ltap = 0, lc = 0;
+    const uint16_t* wl = w;
+    auto load = [&](bf16x8& v) __attribute__((always_inline)) {
+        v = *reinterpret_cast<const bf16x8*>(wl + wlane);
+        lc += 32;
+        wl += 32;
+        if (lc == Cin) {
+            lc = 0;
+            wl += (size_t)(Cout - 1) * Cin;
+            if (++ltap == 9) {
+                ltap = 0;
+                wl = w;
+            }
+        }
+    };
+    auto put = [&](int slot, bf16x8 v) __attribute__((always_inline)) {
+        if (WT == T || wave < WT / 64)
+            *reinterpret_cast<bf16x8*>(&staged[wput + slot * CO * 32]) = v;
+    };
+    // Operands of the next step: its tap and slice (first staged pixel, first
+    // channel), and where the tap's first pixel lies in a slice of either input.
+    const int wread = words + 8 + cl_at(16 * NT * (wave / ROWS) + row, kb);
+    int tap = 0, base = 0, c = 0, full = 0, half = 0;
+    auto place = [&]() __attribute__((always_inline)) {
+        const int y = wave % ROWS + tap / 3, x = row + tap % 3;
+        full = cl_at(y * CT_AX + x, kb);
+        half = cl_at(((y + 1) >> 1) * CT_HX + ((x + 1) >> 1), kb);
+    };
+    place();
+    auto read = [&](int slot, bf16x8 (&a)[4], bf16x8 (&b)[NT]) __attribute__((always_inline)) {
+        const bool first = c < ci.C1, up = first && ci.up1;
+        const int at = (up ? half : full) + base * 32, step = up ? 8 * 32 : 16 * 32;
+#pragma unroll
+        for (int m = 0; m < 4; ++m) a[m] = *reinterpret_cast<const bf16x8*>(&staged[at + m * step]);
+#pragma unroll
+        for (int q = 0; q < NT; ++q)
+            b[q] = *reinterpret_cast<const bf16x8*>(&staged[wread + slot * CO * 32 + 16 * q * 32]);
+        base += first ? np1 : np2;
+        c += 32;
+        if (c == Cin) {
+            c = base = 0;
+            tap = tap < 8 ? tap + 1 : 0;
+            place();
+        }
+    };
+    load(wv[0]);
+    load(wv[1]);
+    if (ci.up1)
+        stage(std::integral_constant<int, CT_HX>(), ci.in1, ci.C1, np1, H / 2, W / 2, y0 / 2 - 1,
+              x0 / 2 - 1, 0);
+    else
+        stage(std::integral_constant<int, CT_AX>(), ci.in1, ci.C1, np1, H, W, y0 - 1, x0 - 1, 0);
+    if (ci.C2)
+        stage(std::integral_constant<int, CT_AX>(), ci.in2, ci.C2, np2, H, W, y0 - 1, x0 - 1,
+              np1 * (ci.C1 / 32));
+    put(0, wv[0]);
+    put(1, wv[1]);
+    load(wv[2]);
+    load(wv[0]);
+    load(wv[1]);
+    f32x4 acc[4][NT];
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+#pragma unroll
+        for (int q = 0; q < NT; ++q) acc[m][q] = f32x4{0.f, 0.f, 0.f, 0.f};
+    __syncthreads();
+    read(0, a[0], b[0]);
+    int slot = 0;  // of the step
+    for (int s = 0; s < 9 * Cin; s += 32 * D) {
+#pragma unroll
+        for (int j = 0; j < D; ++j) {
+            __syncthreads();  // step j + 1's weights are there, j's read
+            // (left to itself the scheduler moves the loads down to their use)
+            read(slot ^ 1, a[(j + 1) % D], b[(j + 1) % D]);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int m = 0; m < 4; ++m)
+#pragma unroll
+                for (int q = 0; q < NT; ++q)
+                    acc[m][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[j][m], b[j][q], acc[m][q], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            put(slot, wv[(j + 2) % D]);
+            load(wv[(j + 2) % D]);
+            slot ^= 1;
         }
     }
+    __syncthreads();  // every wave's operand reads are done
+    conv_out<NT, ROWS, CW, true>(acc, staged, bias, out, outf, fz, n, y0, x0, co0, H, W, Cout, relu);
 }
 
 // Weight gradient of the 3x3 convolution:
@@ -1059,16 +1261,38 @@ int grid_for(long long n) {
 
 }  // namespace
 
-// The LDS-staged convolution is the faster one where output channels come in
-// blocks of 32, unless most of a large launch would be padding: with at least
-// a quarter of its 4 x 64 tiles' pixels in the image (2000 x 24 x 64 -> 64
-// channels: 15 us against 33), or at most two workgroups a CU (8 x 16 x 16:
-// 11 against 32).  On narrower ones the other kernel, whose waves take pixels
-// of several rows, does less.
-inline bool lds_conv_applies(int n, int h, int wdt, int cout) {
+// Tile of k_conv3x3_taps: as many rows as fit into LDS with all channels.
+// rows 0: it does not take the channels, or an odd image with an upsampled
+// input (whose last pixel's second row or column is outside).
+struct TapsTile {
+    int rows, block, cw;
+};
+inline TapsTile conv_taps_tile(int h, int wdt, int c1, int up1, int c2, int cout) {
+    auto fits = [&](int rows, int block, int lds) {
+        return 2 * conv_taps_words(rows, block, c1, up1, c2) <= lds;
+    };
+    if (up1 && (h % 2 || wdt % 2)) return {0, 0, 0};
+    if (cout % 128 == 0 && fits(4, 128, CT_LDS)) return {4, 128, 2};
+    if (cout % 128 == 0 && fits(2, 128, CT_LDS)) return {2, 128, 4};
+    if (cout % 64 == 0 && fits(4, 64, CT_LDS)) return {4, 64, 2};
+    if (cout % 64 != 0 && cout % 32 == 0 && fits(4, 32, CT_LDS)) return {4, 32, 1};
+    return {0, 0, 0};
+}
+inline bool conv_edge(int h, int wdt) { return wdt % CL_TX != 0 || h % 4 != 0; }
+// The LDS-staged convolutions are the faster ones where output channels come
+// in blocks of 32, unless most of a large launch would be padding: with at least
+// a quarter of its 4 x 64 tiles' pixels in the image (2000 rows of 17 pixels,
+// 64 -> 64 channels: 18 us against 32; 8000 rows: 59 against 61), or at most
+// two workgroups a CU (8 images of 16 x 16: 12 against 31).  On narrower ones
+// the other kernel, whose waves take pixels of several rows, does less.
+inline bool lds_conv_applies(int n, int h, int wdt, int c1, int up1, int c2, int cout) {
+    // (k_conv3x3_lds numbers the pixels in 32 bits)
+    if (cout % 32 != 0 || (long long)n * h * wdt > INT32_MAX) return false;
+    if (conv_edge(h, wdt) && c1 + c2 > 32 && conv_taps_tile(h, wdt, c1, up1, c2, cout).rows == 0)
+        return false;
     const long long tiles = (long long)n * ((h + 3) / 4) * ((wdt + CL_TX - 1) / CL_TX);
-    return cout % 32 == 0 && (4LL * n * h * wdt >= tiles * 4 * CL_TX ||
-                              tiles * (cout % 64 == 0 ? cout / 64 : cout / 32) <= 512);
+    return 4LL * n * h * wdt >= tiles * 4 * CL_TX ||
+           tiles * (cout % 64 == 0 ? cout / 64 : cout / 32) <= 512;
 }
 // Output channels of one workgroup of the LDS-staged convolution.
 inline int lds_conv_block(int cout) { return cout % 64 == 0 ? 64 : 32; }
@@ -1083,18 +1307,29 @@ int launch_conv_lds(void* stream, const ConvIn& ci, const uint16_t* w, const flo
                     uint16_t* out, float* outf, const ConvFuse& fz, int n, int h, int wdt, int cout,
                     int relu) {
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    const unsigned tiles = (unsigned)n * ((h + 3) / 4) * ((wdt + CL_TX - 1) / CL_TX);
-    auto launch = [&](auto kernel, int block) {
-        hipLaunchKernelGGL(kernel, dim3(tiles, cout / block), dim3(256), 0, st, ci, w, bias, out,
+    const bool edge = conv_edge(h, wdt), taps = edge && ci.C1 + ci.C2 > 32;
+    const TapsTile tile = taps ? conv_taps_tile(h, wdt, ci.C1, ci.up1, ci.C2, cout) : TapsTile{4, 0, 0};
+    if (tile.rows == 0) return CAGEO_ERR_ARG;
+    const unsigned tiles = (unsigned)n * ((h + tile.rows - 1) / tile.rows) * ((wdt + CL_TX - 1) / CL_TX);
+    auto launch = [&](auto kernel, int block, int threads, size_t lds) {
+        hipLaunchKernelGGL(kernel, dim3(tiles, cout / block), dim3(threads), lds, st, ci, w, bias, out,
                            outf, fz, n, h, wdt, cout, relu);
     };
-    const bool edge = wdt % CL_TX != 0 || h % 4 != 0;
-    if (cout % 64 == 0) {
-        if (edge) launch(k_conv3x3_lds<4, 1, 2, true>, 64);
-        else launch(k_conv3x3_lds<4, 1, 2, false>, 64);
+    if (taps) {
+        auto taps_of = [&](auto kernel, int out_words) {
+            const int words = conv_taps_words(tile.rows, tile.block, ci.C1, ci.up1, ci.C2);
+            launch(kernel, tile.block, 64 * tile.rows * tile.cw, 2 * (size_t)std::max(words, out_words));
+        };
+        if (tile.rows == 2) taps_of(k_conv3x3_taps<2, 2, 4>, conv_out_words<2, 2, 4>());
+        else if (tile.block == 128) taps_of(k_conv3x3_taps<4, 4, 2>, conv_out_words<4, 4, 2>());
+        else if (tile.cw == 2) taps_of(k_conv3x3_taps<2, 4, 2>, conv_out_words<2, 4, 2>());
+        else taps_of(k_conv3x3_taps<2, 4, 1>, conv_out_words<2, 4, 1>());
+    } else if (cout % 64 == 0) {
+        if (edge) launch(k_conv3x3_lds<4, 2, true>, 64, 256, 0);
+        else launch(k_conv3x3_lds<4, 2, false>, 64, 256, 0);
     } else {
-        if (edge) launch(k_conv3x3_lds<2, 1, 3, true>, 32);
-        else launch(k_conv3x3_lds<2, 1, 3, false>, 32);
+        if (edge) launch(k_conv3x3_lds<2, 3, true>, 32, 256, 0);
+        else launch(k_conv3x3_lds<2, 3, false>, 32, 256, 0);
     }
     CAGEO_HIP_TRY(hipGetLastError());
     return CAGEO_OK;
@@ -1177,7 +1412,7 @@ bool nn_conv3x3_fused(void* stream, const uint16_t* in1, int c1, int up1, const 
                       int c2, const uint16_t* w, const float* bias, uint16_t* out, uint16_t* pool,
                       const float* head_w, const float* head_b, float* prob, int head_sigmoid,
                       int n, int h, int wdt, int cout, int relu, int* status) {
-    if (!lds_conv_applies(n, h, wdt, cout) || (pool && (h % 2 || wdt % 2)) ||
+    if (!lds_conv_applies(n, h, wdt, c1, up1, c2, cout) || (pool && (h % 2 || wdt % 2)) ||
         (prob && lds_conv_block(cout) != cout))
         return false;
     const ConvIn ci{in1, in2, c1, c2, up1};
@@ -1200,7 +1435,7 @@ int cageo_nn_conv3x3(void* stream, const uint16_t* in1, int c1, int up1, const u
     if (c1 <= 0 || c1 % 32 || c2 < 0 || c2 % 32 || (c2 && !in2) || cout % 16) return CAGEO_ERR_ARG;
     ConvIn ci{in1, in2, c1, c2, up1};
     const long long M = (long long)n * h * wdt;
-    if (lds_conv_applies(n, h, wdt, cout))
+    if (lds_conv_applies(n, h, wdt, c1, up1, c2, cout))
         return launch_conv_lds(stream, ci, w, bias, out, outf, ConvFuse{}, n, h, wdt, cout, relu);
     // output channel tile: 64 (NT 4), 32 (NT 2) or 16 (NT 1); 4 pixel tiles
     // per wave (256 pixels per workgroup; 8 lowered occupancy and time)
