@@ -11,13 +11,15 @@
 //             every tile, then ONE pit-fill, ONE flow-routing and ONE
 //             flow-tracing launch over the 64x64 blocks of all tiles at once
 //             (the persistent kernels take a table of rasters), then the
-//             border accumulation of every tile; all on one stream, one wait;
+//             border accumulation of every tile; the per-tile launches of
+//             tiles that share nothing run beside each other, one wait;
 //   GRAPH     that sequence for one realization captured once as a hipGraph
 //             and replayed n times; the random-field kernels read the
 //             realization index from device memory, which a last node bumps.
 // A small tile has few 64x64 blocks, so its own persistent launch leaves most
-// of the chip idle while it iterates; in one launch over all tiles the number
-// of barrier-separated passes is that of the slowest tile, not the sum.
+// of the chip idle while it iterates; in one launch over all tiles their
+// dependent steps (the pit fill's chains of tile visits, the flats' passes)
+// run beside each other, and the slowest tile's decide, not the sum.
 // The autotuner picks, per tile, the workgroup count of its own persistent
 // launches and the row-block height of the 2-D convolution, and then the
 // workgroup count of the all-tile launches.
@@ -101,14 +103,47 @@ int ensure_multi(cageo_batch* b) {
     return CAGEO_OK;
 }
 
+// Streams of the per-tile launches, by tile: 0 the batch's, i side[i - 1].
+// Before the all-tile launches the tiles share nothing and take the streams
+// in turn.  The border launches add to the counters by a load and a store, so
+// tiles whose counter rasters overlap (several error models summed into one
+// map) follow each other on one stream.
+struct TileStreams {
+    std::vector<int> pre, border;
+};
+TileStreams tile_streams(const cageo_batch* b, float* const* mc) {
+    const int T = (int)b->tiles.size(), streams = std::min(T, cageo_batch::SIDES + 1);
+    TileStreams s;
+    std::vector<int> order, set(T), stream_of(T, -1);
+    for (int t = 0; t < T; ++t) {
+        s.pre.push_back(t % streams);
+        set[t] = t;
+        if (mc[t]) order.push_back(t);
+    }
+    std::sort(order.begin(), order.end(), [&](int a, int c) { return (uintptr_t)mc[a] < (uintptr_t)mc[c]; });
+    uintptr_t end = 0;  // of the counters of the present set
+    for (size_t i = 0; i < order.size(); ++i) {
+        const int t = order[i];
+        const uintptr_t at = (uintptr_t)mc[t];
+        if (i > 0 && at < end) set[t] = set[order[i - 1]];
+        end = std::max(end, at + b->tiles[t].ctx->c.n * sizeof(float));
+    }
+    int sets = 0;
+    for (int t = 0; t < T; ++t) {
+        int& k = stream_of[set[t]];
+        if (k < 0) k = sets++ % streams;
+        s.border.push_back(k);
+    }
+    return s;
+}
+
 // fn(t, context) for every tile, whose launches go to the context's stream:
-// the tiles take the batch's stream and the side streams in turn, forked from
-// the batch's and joined to it, so that the launches of small tiles run
-// beside each other (a 256 to 1024 cells wide tile fills a part of the
-// device only).  A realization of 12 such tiles: 1.67 ms, 2.08 with all of
-// them on one stream.
+// stream[t] (see TileStreams), the side streams forked from the batch's and
+// joined to it, so that the launches of small tiles run beside each other (a
+// 256 to 1024 cells wide tile fills a part of the device only).  A realization
+// of 12 such tiles: 1.67 ms, 2.08 with all of them on one stream.
 template <class F>
-int each_tile(cageo_batch* b, F fn) {
+int each_tile(cageo_batch* b, const std::vector<int>& stream, F fn) {
     const int T = (int)b->tiles.size();
     const int sides = std::min(T - 1, (int)cageo_batch::SIDES);
     if (sides > 0) CAGEO_HIP_TRY(hipEventRecord(b->fork, b->stream));
@@ -116,8 +151,7 @@ int each_tile(cageo_batch* b, F fn) {
     int st = CAGEO_OK;
     for (int t = 0; t < T && st == CAGEO_OK; ++t) {
         Context* c = &b->tiles[t].ctx->c;
-        const int i = t % (sides + 1);
-        if (i > 0) c->stream = b->side[i - 1];
+        if (stream[t] > 0) c->stream = b->side[stream[t] - 1];
         st = fn(t, c);
         c->stream = b->stream;
     }
@@ -129,8 +163,9 @@ int each_tile(cageo_batch* b, F fn) {
 }
 
 // One realization of every tile with the all-tile persistent launches.
-int enqueue_all(cageo_batch* b, float* const* mc, uint32_t first, const uint32_t* base) {
-    CAGEO_TRY(each_tile(b, [&](int t, Context* c) -> int {
+int enqueue_all(cageo_batch* b, float* const* mc, const TileStreams& ts, uint32_t first,
+                const uint32_t* base) {
+    CAGEO_TRY(each_tile(b, ts.pre, [&](int t, Context* c) -> int {
         CAGEO_TRY(launch_random_field(c, c->d_a, b->tiles[t].seed, first, 0u, c->mean,
                                       c->std_dev, base));
         return realization_pre(c, nullptr);
@@ -138,7 +173,7 @@ int enqueue_all(cageo_batch* b, float* const* mc, uint32_t first, const uint32_t
     CAGEO_TRY(pit_fill_multi(&b->multi, b->stream));
     CAGEO_TRY(flow_routing_multi(&b->multi, b->stream));
     CAGEO_TRY(flow_tracing_multi(&b->multi, b->stream));
-    return each_tile(b, [&](int t, Context* c) -> int {
+    return each_tile(b, ts.border, [&](int t, Context* c) -> int {
         return mc[t] ? launch_border(c, mc[t], c->d_lab) : CAGEO_OK;
     });
 }
@@ -167,9 +202,10 @@ int build_graph(cageo_batch* b, float* const* mc) {
     // tables and workgroup counts are fixed before capture (no allocations or
     // device queries inside it)
     CAGEO_TRY(ensure_multi(b));
+    const TileStreams ts = tile_streams(b, mc);
     hipGraph_t g = nullptr;
     CAGEO_HIP_TRY(hipStreamBeginCapture(b->stream, hipStreamCaptureModeRelaxed));
-    int st = enqueue_all(b, mc, 0u, b->d_iter);
+    int st = enqueue_all(b, mc, ts, 0u, b->d_iter);
     if (st == CAGEO_OK) {
         hipLaunchKernelGGL(k_bump_u32, dim3(1), dim3(64), 0, b->stream, b->d_iter);
         if (hipGetLastError() != hipSuccess) st = CAGEO_ERR_HIP;
@@ -207,8 +243,9 @@ int time_tile(cageo_batch* b, int t, float* mc, int reps, float* ms) {
 int time_all(cageo_batch* b, float* const* mc, int reps, float* ms) {
     Context* c = &b->tiles[0].ctx->c;
     hipEvent_t e0 = c->ev[0], e1 = c->ev[1];
+    const TileStreams ts = tile_streams(b, mc);
     CAGEO_HIP_TRY(hipEventRecord(e0, b->stream));
-    for (int r = 0; r < reps; ++r) CAGEO_TRY(enqueue_all(b, mc, (uint32_t)r, nullptr));
+    for (int r = 0; r < reps; ++r) CAGEO_TRY(enqueue_all(b, mc, ts, (uint32_t)r, nullptr));
     CAGEO_HIP_TRY(hipEventRecord(e1, b->stream));
     CAGEO_HIP_TRY(hipEventSynchronize(e1));
     CAGEO_TRY(check_all(b));
@@ -391,7 +428,9 @@ int cageo_batch_run(cageo_batch* b, float* const* d_mc, int n, uint32_t first, i
         return CAGEO_OK;
     }
     if (mode == CAGEO_BATCH_STREAM) {
-        for (int r = 0; r < n; ++r) CAGEO_TRY(cageo::enqueue_all(b, d_mc, first + (uint32_t)r, nullptr));
+        const cageo::TileStreams ts = cageo::tile_streams(b, d_mc);
+        for (int r = 0; r < n; ++r)
+            CAGEO_TRY(cageo::enqueue_all(b, d_mc, ts, first + (uint32_t)r, nullptr));
         return cageo::check_all(b);
     }
     if (mode != CAGEO_BATCH_GRAPH) return CAGEO_ERR_ARG;

@@ -218,10 +218,11 @@ int cageo_stage_times(cageo_context* ctx, float* out, int enable);
  * realization r computes exactly what cageo_run_realizations does on that
  * tile alone, in every mode:
  *   CAGEO_BATCH_PER_TILE  one blocking cageo_run_realizations per tile;
- *   CAGEO_BATCH_STREAM    all tiles x realizations on one stream, one wait;
+ *   CAGEO_BATCH_STREAM    all tiles x realizations enqueued, one wait;
  *   CAGEO_BATCH_GRAPH     one realization of all tiles captured as a hipGraph
  *                         and replayed n times.
- * d_mc is an array of ntiles device pointers (one counter raster per tile).
+ * d_mc is an array of ntiles device pointers, one counter raster per tile;
+ * they may be the same for several tiles, which then add to one map.
  * With hip_stream NULL the batch creates its own (blocking, default-priority)
  * stream, since the NULL stream cannot be captured into a graph. */
 #define CAGEO_BATCH_PER_TILE 0
