@@ -19,8 +19,8 @@
 //      (256 slots per tile);
 //   2. over the border table only: exits jump through the entries of the
 //      slots they name, in place, until no exit is left; a chain of more
-//      steps than the raster has cells, or of more hops than there are slots,
-//      is a cycle through several tiles (stuck).  In place, and without
+//      steps than the raster has cells (or an entry holds), or of more hops
+//      than there are slots, is a cycle through several tiles (stuck).  In place, and without
 //      waiting for each other, is safe because every entry of a slot, old or
 //      rewritten, names a slot on that cell's own path with the step count to
 //      it, so a hop through either is correct, and a rewritten one is further
@@ -36,13 +36,12 @@
 #include <vector>
 
 #include "common.hpp"
+#include "trace_steps.hpp"
 
 namespace cageo {
 
 namespace {
 
-constexpr uint32_t K_LOCAL = 0, K_RESOLVED = 1, K_EXIT = 2, K_STUCK = 3;
-constexpr uint64_t STEP_MASK = (1ull << 30) - 1;
 constexpr int BORDER_SLOTS = 256;
 
 // Slot of tile cell (lx, ly) in its tile's border table: row 0 -> 0..63,
@@ -54,23 +53,6 @@ __device__ inline int border_slot(int lx, int ly) {
     s = lx == 0 ? 2 * TILE + ly : s;
     s = ly == TILE - 1 ? TILE + lx : s;
     return ly == 0 ? lx : s;
-}
-
-__device__ inline uint64_t pack(uint32_t kind, uint32_t steps, int32_t value) {
-    return ((uint64_t)kind << 62) | ((uint64_t)(steps & STEP_MASK) << 32) |
-           (uint64_t)(uint32_t)value;
-}
-__device__ inline uint32_t kind_of(uint64_t e) { return (uint32_t)(e >> 62); }
-__device__ inline uint32_t steps_of(uint64_t e) { return (uint32_t)((e >> 32) & STEP_MASK); }
-__device__ inline int32_t value_of(uint64_t e) { return (int32_t)(uint32_t)e; }
-
-// Follow entry e one hop through entry f (the entry of e's target).
-__device__ inline uint64_t hop(uint64_t e, uint64_t f) {
-    uint32_t s = steps_of(e) + steps_of(f);
-    if (s > STEP_MASK) s = STEP_MASK;
-    const uint32_t k = kind_of(f);
-    if (k == K_STUCK) return pack(K_STUCK, 0, 0);
-    return pack(k, s, value_of(f));
 }
 
 // Pointer of a cell within its tile: kind (2 bits) | steps (16 bits,
@@ -349,7 +331,7 @@ __global__ __launch_bounds__(256) void k_tr_jump(TrArgs a) {
             if (kind_of(e) == K_EXIT) {
                 uint64_t ne = hop(e, ld64(&tb[value_of(e)]));
                 if (kind_of(ne) == K_EXIT) {
-                    if (steps_of(ne) > (uint32_t)b.R.W * (uint32_t)b.R.H || rounds > slots)
+                    if (is_cycle(steps_of(ne), (uint32_t)b.R.W * (uint32_t)b.R.H) || rounds > slots)
                         ne = pack(K_STUCK, 0, 0);
                     else
                         pending = true;
