@@ -670,7 +670,11 @@ constexpr int WG_XROW = 32 * WG_XS;
 __device__ inline uint32_t pair_lo(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x05040100u); }
 __device__ inline uint32_t pair_hi(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302u); }
 
-template <int CO>
+// EDGE: W % 64 or H % 2.  Beyond the right edge and below the last row g is
+// staged as zeros; x is not zero there for the taps that move the last pixel
+// or row in, and may be infinite, so those products are left out (2 to 12 % of
+// such a launch).
+template <int CO, bool EDGE>
 __global__ __launch_bounds__(WG_T) __attribute__((amdgpu_waves_per_eu(4))) void k_conv3x3_wgrad(
     ConvIn ci, const uint16_t* __restrict__ g, float* __restrict__ dw, int N, int H, int W, int Cout,
     int rows) {
@@ -791,7 +795,7 @@ __global__ __launch_bounds__(WG_T) __attribute__((amdgpu_waves_per_eu(4))) void 
         const bool more = y + 2 < y1;
         if (more) load(y + 3, y + 2);
         const uint16_t* gr = gt + (2 * buf + wrow) * GROW + (32 * wco + row) * WG_GS + 8 * kb;
-        for (int c = c_lo; c < c_hi; ++c) {
+        for (int c = EDGE && y + wrow >= y1 ? c_hi : c_lo; c < c_hi; ++c) {
             bf16x8 a[2];
 #pragma unroll
             for (int q = 0; q < 2; ++q)
@@ -809,7 +813,18 @@ __global__ __launch_bounds__(WG_T) __attribute__((amdgpu_waves_per_eu(4))) void 
                 const uint32_t s2 = __builtin_amdgcn_alignbit(m.z, m.y, 16);
                 const uint32_t s3 = __builtin_amdgcn_alignbit(m.w, m.z, 16);
                 const uint32_t s4 = __builtin_amdgcn_alignbit(nx, m.w, 16);
-                const bf16x8 b0 = as_bf16x8(make_uint4(s0, s1, s2, s3));  // pixel - 1
+                uint4 u0 = make_uint4(s0, s1, s2, s3);  // pixel - 1
+                if (EDGE && (uint32_t)(W - x0 - 32 * c) < 32u) {
+                    int end = W - x0 - 32 * c;
+                    asm volatile("" : "+s"(end));  // (masks kept for the three rows would spill)
+                    const int e = end - 8 * kb;
+                    const uint32_t keep = (e & 1) ? 0xffffu : 0xffff0000u;
+                    if (e >> 1 == 0) u0.x &= keep;
+                    if (e >> 1 == 1) u0.y &= keep;
+                    if (e >> 1 == 2) u0.z &= keep;
+                    if (e >> 1 == 3) u0.w &= keep;
+                }
+                const bf16x8 b0 = as_bf16x8(u0);
                 const bf16x8 b1 = as_bf16x8(m);
                 const bf16x8 b2 = as_bf16x8(make_uint4(s1, s2, s3, s4));  // pixel + 1
 #pragma unroll
@@ -1492,12 +1507,14 @@ int cageo_nn_conv3x3_wgrad(void* stream, const uint16_t* in1, int c1, int up1,
     const dim3 grid((unsigned)(segs * n * ((h + rows - 1) / rows)), (unsigned)(cout / co),
                     (unsigned)((c1 + c2) / 32));
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    if (co == 64)
-        hipLaunchKernelGGL(k_conv3x3_wgrad<64>, grid, dim3(WG_T), 0, st, ci, g, dw, n, h, wdt, cout,
-                           (int)rows);
-    else
-        hipLaunchKernelGGL(k_conv3x3_wgrad<32>, grid, dim3(WG_T), 0, st, ci, g, dw, n, h, wdt, cout,
-                           (int)rows);
+    const bool edge = wdt % 64 != 0 || h % 2 != 0;
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(WG_T), 0, st, ci, g, dw, n, h, wdt, cout, (int)rows);
+    };
+    if (co == 64 && edge) launch(k_conv3x3_wgrad<64, true>);
+    else if (co == 64) launch(k_conv3x3_wgrad<64, false>);
+    else if (edge) launch(k_conv3x3_wgrad<32, true>);
+    else launch(k_conv3x3_wgrad<32, false>);
     CAGEO_HIP_TRY(hipGetLastError());
     return CAGEO_OK;
 }
