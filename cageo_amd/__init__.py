@@ -345,7 +345,8 @@ class Trainer:
     """Training of the border-probability surrogate behind the C ABI
     (cageo_trainer, cageo_surrogate_train): fp32 master weights, Adam, the
     forward and backward passes on the library's BF16 MFMA kernels.
-    Inputs are fp32 device tensors [tiles][h][w][4], targets [tiles][h][w]."""
+    Inputs are fp32 device tensors [tiles][h][w][4], targets [tiles][h][w].
+    Base 32 trains; 64, 96 and 128 only hold, read and save their weights."""
 
     def __init__(self, base=32, seed=0, init_weights=None, stream=None):
         h = ctypes.c_void_p()

@@ -306,12 +306,14 @@ int layer_back(cageo_trainer* t, int i, const uint16_t* g, int prev, uint16_t* g
     return CAGEO_OK;
 }
 
+// The bases that train: the head's backward pass and the bias sums take 32 to
+// 256 channels in powers of two, and the middle layers have 8 x base.
+bool trains(const cageo_trainer* t) { return t->base == 32; }
+
 // Backward pass after forward(): parameter gradients (zeroed first) and the
 // batch's mean BCE added to *d_loss.
 int backward(cageo_trainer* t, float* d_loss) {
     const int b = t->base, n = t->n, h = t->h, w = t->w;
-    // the bias sums take power-of-two channel counts up to 256
-    if (b != 32) return CAGEO_ERR_ARG;
     void* s = t->stream;
     const auto& A = t->act;
     float* const* DC = t->gr.data();      // of the concatenated inputs of D1A, D2A, D3A
@@ -598,7 +600,8 @@ int cageo_trainer_create(cageo_trainer** out, int base, uint64_t seed, const cha
 
 int cageo_trainer_gradients(cageo_trainer* t, const float* d_x, const float* d_target, int n,
                             int h, int w, float* loss) {
-    if (!t || !d_x || !d_target || n <= 0 || h <= 0 || w <= 0 || h % 8 || w % 8)
+    if (!t || !d_x || !d_target || n <= 0 || h <= 0 || w <= 0 || h % 8 || w % 8 ||
+        !cageo::trains(t))
         return CAGEO_ERR_ARG;
     CAGEO_TRY(cageo::ensure_batch(t, n, h, w));
     CAGEO_TRY(cageo::ensure_loop(t, 1, 2LL * n));
@@ -635,6 +638,7 @@ int cageo_surrogate_train(cageo_trainer* t, const float* d_x, const float* d_y, 
         nsteps < 0 || first_step < 0 || total_steps < first_step + nsteps || !(lr > 0.0f))
         return CAGEO_ERR_ARG;
     if (nsteps == 0) return CAGEO_OK;
+    if (!cageo::trains(t)) return CAGEO_ERR_ARG;
     CAGEO_TRY(cageo::ensure_batch(t, batch, h, w));
     CAGEO_TRY(cageo::ensure_loop(t, nsteps, 2LL * batch * nsteps));
     // every step's batch, drawn from the step number (a run in pieces draws

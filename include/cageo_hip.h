@@ -417,8 +417,10 @@ int cageo_surrogate_check(cageo_surrogate* s, cageo_context* ctx, const float* d
 /* ---- border-probability surrogate: training --------------------------------
  * No reference counterpart (the reference has no learned part).  A trainer
  * holds the network's fp32 master weights, their bf16 copies, gradients
- * and Adam moments (beta 0.9 / 0.999, eps 1e-8) for base `base` (a multiple
- * of 32), and the workspace of one batch shape.  Initial weights: the
+ * and Adam moments (beta 0.9 / 0.999, eps 1e-8) for base `base` (32, 64, 96
+ * or 128; base 32 trains, the others only hold, read and save their weights,
+ * and their gradient, step and train calls return CAGEO_ERR_ARG), and the
+ * workspace of one batch shape.  Initial weights: the
  * weights file `init_weights` (surrogate format; NULL: He-normal from
  * `seed`, zero biases).  Inputs are fp32 NHWC [tiles][h][w][4] (z-scored
  * DEM, stream mask 0/1, RMSE / 3 m, practical range / 200 m; h, w multiples

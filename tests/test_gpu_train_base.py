@@ -24,7 +24,7 @@ def test_other_bases_are_refused_at_once(torch_cuda, tmp_path, base):
                 call()
             assert err.value.status == -1
         torch.cuda.synchronize()
-        # (the workspace of four tiles of 256^2 takes 1 GB and more)
+        # (the workspace of four tiles of 256^2 takes 365 MB and more)
         assert torch.cuda.mem_get_info()[0] >= free - (64 << 20)
         path = str(tmp_path / "w.bin")
         tr.save(path)
