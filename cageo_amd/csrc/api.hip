@@ -81,7 +81,7 @@ int realization_body(Context* c, float* mc, hipEvent_t* evs) {
     };
     CAGEO_TRY(realization_pre(c, evs));
     ev = 4;
-    CAGEO_TRY(pit_fill_quantized(c, c->d_z, c->d_w, c->nodata_dem, true));
+    CAGEO_TRY(pit_fill_quantized(c, c->d_z, c->d_w, c->nodata_dem));
     CAGEO_TRY(mark());
     CAGEO_TRY(flow_routing(c, c->d_w, c->d_fd));
     CAGEO_TRY(mark());
@@ -406,7 +406,7 @@ int cageo_pit_fill(cageo_context* ctx, float* d_filled, float* d_dem, float noda
     CAGEO_TRY(cageo::clear_status(c));
     CAGEO_TRY(cageo::reset_minmax(c));
     CAGEO_TRY(cageo::launch_quantize(c, d_dem, nodata));
-    CAGEO_TRY(cageo::pit_fill_quantized(c, d_dem, d_filled, nodata, true));
+    CAGEO_TRY(cageo::pit_fill_quantized(c, d_dem, d_filled, nodata));
     return cageo::check_status(c);
 }
 

@@ -345,8 +345,6 @@ enum : int {
     CTL_EPOCH = 7,      // epoch counter of the pit-fill worklists
     CTL_ROUNDS = 8,
     CTL_PASSES = 9,
-    CTL_FLAG = 10,      // 3 words, free (pass-end flags travel with the barrier)
-    CTL_EPOCH_FR = 13,  // free (flat-resolution epochs start over each launch)
     CTL_FR_PASSES = 14, // flat-resolution passes of the last launch
     CTL_TR_ROUNDS = 15, // exit-jump rounds of the last tracing launch
     CTL_PHASE = 16,     // 3 phase-list counts (pit fill)
@@ -450,7 +448,7 @@ int launch_stream_flags(Context* c, const float* stream, float nodata_stream, ui
                         int32_t* slabel);
 int launch_realistic_burn_quant(Context* c, const float* dem, const float* e, float* zq);
 size_t burn_blocks(int W, int H);
-int pit_fill_quantized(Context* c, float* zq, float* w, float nodata, bool stats_ready);
+int pit_fill_quantized(Context* c, float* zq, float* w, float nodata);
 int check_status(Context* c);
 int reset_minmax(Context* c);
 // One realization from the error field in c->d_a (stages a3..a9); with

@@ -62,13 +62,13 @@ struct FrRaster {
     int W, H, ntx, nty;
 };
 
-// A launch over one raster (`one`, rs null) or over the nr rasters of a
+// A launch over one raster (`one`, rs null) or over the rasters of a
 // table, whose 64x64 blocks are numbered globally (bmap).
 struct FrArgs {
     FrRaster one;
     const FrRaster* __restrict__ rs;
     const int2* __restrict__ bmap;  // per block: (raster, block within it)
-    int nr, total;
+    int total;
     int* work;      // 3 lists of `total` entries
     uint32_t* mark; // per-block epoch stamps
     Row64* nbr;     // per block: the other 4 directions x 64 rows
@@ -761,7 +761,6 @@ int flow_routing(Context* c, const float* z, int8_t* fd) {
     a.one = fr_raster(c, z, fd);
     a.rs = nullptr;
     a.bmap = nullptr;
-    a.nr = 1;
     a.total = c->ntiles;
     a.work = c->d_work3;
     a.mark = c->d_mark;
@@ -771,7 +770,7 @@ int flow_routing(Context* c, const float* z, int8_t* fd) {
     a.max_passes = 1 << 20;
     hipLaunchKernelGGL(k_fr_reset, dim3((a.total + 255) / 256), dim3(256), 0, c->stream, a);
     hipLaunchKernelGGL(k_fr_d8<false>, dim3(a.total), dim3(TILE_THREADS), 0, c->stream, a);
-    // ordinary launch within the occupancy cap (see pit_fill_quantized); no
+    // ordinary launch within the occupancy cap (see pf_launch); no
     // more workgroups than blocks, as each adds to the barriers (the routing
     // of 1000 x 777, 208 blocks: 226 us, 277 with the full grid)
     hipLaunchKernelGGL(k_fr_persistent<false>, dim3(std::min(c->fr_grid, a.total)),
@@ -805,7 +804,6 @@ int flow_routing_multi(MultiState* m, hipStream_t s) {
     a.one = FrRaster{};
     a.rs = static_cast<const FrRaster*>(m->d_fr);
     a.bmap = m->d_bmap;
-    a.nr = m->nr;
     a.total = m->total;
     a.work = m->d_work;
     a.mark = m->d_mark_fr;

@@ -243,13 +243,13 @@ struct TrRaster {
     uint32_t* scal;
 };
 
-// A launch over one raster (`one`, rs null) or over the nr rasters of a
+// A launch over one raster (`one`, rs null) or over the rasters of a
 // table, whose 64x64 blocks are numbered globally (bmap).
 struct TrArgs {
     TrRaster one;
     const TrRaster* __restrict__ rs;
     const int2* __restrict__ bmap;  // per block: (raster, block within it)
-    int nr, total;
+    int total;
     uint32_t* ctrl;
     GridBar gb;     // status and abort words (no barrier is used)
 };
@@ -436,7 +436,6 @@ int flow_tracing(Context* c, const int8_t* fd, const uint8_t* sflags, const int3
     a.one = tr_raster(c, fd, sflags, slabel, lab);
     a.rs = nullptr;
     a.bmap = nullptr;
-    a.nr = 1;
     a.total = c->ntiles;
     a.ctrl = c->d_ctrl;
     a.gb = context_gridbar(c);
@@ -472,7 +471,6 @@ int flow_tracing_multi(MultiState* m, hipStream_t s) {
     a.one = TrRaster{};
     a.rs = static_cast<const TrRaster*>(m->d_tr);
     a.bmap = m->d_bmap;
-    a.nr = m->nr;
     a.total = m->total;
     a.ctrl = m->d_ctrl;
     a.gb = multi_gridbar(m);

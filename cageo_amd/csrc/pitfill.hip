@@ -719,9 +719,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
             T.lower = false;
         }
         // Visits: first one to each of the workgroup's tiles that the stage
-        // concerns, then those the neighbours ask for.  One body for both (and
+        // concerns, then those the neighbours ask for.  One body for both, and
         // so one copy of the sweeps: with three the loop outgrew the
-        // instruction cache and 280 scalars went to vector registers).
+        // instruction cache.  (The compiler keeps 293 of its scalars in vector
+        // registers; in the table form 275, with 10 vector registers in
+        // scratch.)
         uint32_t ahead = 0;
         bool began = false;
         for (;;) {
@@ -978,7 +980,7 @@ int pit_fill_persistent_grid(Context* c, int* grid) {
     return CAGEO_OK;
 }
 
-int pit_fill_quantized(Context* c, float* zq, float* w, float nodata, bool /*stats_ready*/) {
+int pit_fill_quantized(Context* c, float* zq, float* w, float nodata) {
     int grid = 0;
     CAGEO_TRY(pit_fill_persistent_grid(c, &grid));
     PfArgs a;

@@ -82,7 +82,6 @@ constexpr int BT_X = 64, BT_R = 8, BT_Y = 4 * BT_R;
 constexpr int BH_MAX = CAGEO_MAX_BEVEL_RADIUS;
 constexpr int BE_Y = BT_Y + 2 * BH_MAX;  // rows of a block with its halo
 static_assert(BH_MAX <= 8, "the 2R side cells of a row take 16 bits");
-static_assert(BT_R + 2 * BH_MAX <= 64, "a row of a wave's windows a lane");
 typedef unsigned long long Mask64;
 
 // REAL: the tile's values are realistic_value(z0, z1) (the fused Monte
