@@ -62,8 +62,7 @@ STAGE_BYTES = {
 }
 STAGE_NAMES = ["random_field", "convolution", "realistic_burn", "pit_fill", "flow_routing",
                "flow_tracing", "border"]
-# The kernel launches each stage's events bracket (the pit fill's resident
-# kernel ends at once when the first kernel converged alone).
+# The kernels of each stage's launches.
 STAGE_KERNEL = {
     "random_field": ("k_random_field",), "realistic_burn": ("k_realistic_burn_quant",),
     "pit_fill": ("k_pf_start", "k_pf_fill"),

@@ -41,7 +41,7 @@ LAKE = -9998
 _STATUS = {0: "ok", -1: "invalid argument", -2: "HIP runtime error",
            -3: "device allocation failed", -4: "iteration cap reached",
            -5: "invalid call order", -6: "input outside the supported domain",
-           -7: "persistent launch abandoned (abort word or barrier time limit)"}
+           -7: "persistent launch abandoned (abort word or time limit of a wait)"}
 ERR_ABORTED = -7
 
 # Every live handle (context, batch, surrogate), closed before the interpreter
@@ -578,7 +578,7 @@ class Context:
 
     def abort(self, set_=True):
         """Raise (or clear) the abort word: while it is raised, persistent
-        launches end at their start, or in a barrier wait that stalls, with
+        launches end at their start, or in a wait that stalls, with
         CAGEO_ERR_ABORTED."""
         _check(lib().cageo_context_abort(self._h, int(bool(set_))), "context_abort")
 

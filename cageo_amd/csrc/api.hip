@@ -207,7 +207,7 @@ const char* cageo_status_string(int s) {
         case CAGEO_ERR_NOT_CONVERGED: return "iteration cap reached";
         case CAGEO_ERR_STATE: return "invalid call order";
         case CAGEO_ERR_RANGE: return "input outside the supported domain";
-        case CAGEO_ERR_ABORTED: return "persistent launch abandoned (abort word or barrier time limit)";
+        case CAGEO_ERR_ABORTED: return "persistent launch abandoned (abort word or time limit of a wait)";
         default: return "unknown status";
     }
 }

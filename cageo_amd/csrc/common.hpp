@@ -164,7 +164,9 @@ __host__ __device__ inline bool pf_live(float v, float min_elev) {
     return pf_to_elev(pf_to_index(v, min_elev), min_elev) == v;
 }
 
-// Grid-wide barrier of the persistent kernels.  All workgroups must be
+// Grid-wide barrier of the flat passes and of the pit fill by rounds (the pit
+// fill by bounds waits for other workgroups in its own way and shares the
+// bound and the abort words; the tracing waits for none).  All workgroups must be
 // co-resident: the grids are capped at the device's occupancy limit for the
 // kernel, so every workgroup runs at once when the device is free of other
 // work (other work can only delay a workgroup's start, and the barrier then
@@ -232,7 +234,8 @@ constexpr double BAR_DEFAULT_TIMEOUT_S = 5.0;
 struct GridBar {
     uint32_t* bar;                // BAR_WORDS device words
     const uint32_t* host_abort;   // host-mapped word raised by the host (may be null)
-    uint64_t limit;               // bound of one wait, in wall_clock64() ticks
+    uint64_t limit;               // bound of one wait (of the pit fill by bounds: without any
+                                  // workgroup's progress), in wall_clock64() ticks
     uint32_t* status;             // the launch's sticky status word
 };
 
@@ -346,7 +349,7 @@ enum : int {
     CTL_ROUNDS = 8,
     CTL_PASSES = 9,
     CTL_FR_PASSES = 14, // flat-resolution passes of the last launch
-    CTL_TR_ROUNDS = 15, // exit-jump rounds of the last tracing launch
+    CTL_TR_ROUNDS = 15, // most exit jumps of a chain of the last tracing launch
     CTL_PHASE = 16,     // 3 phase-list counts (pit fill)
     CTL_CLAIM = 19,     // 3 rotating tile-claim counters of the passes
     CTL_COMPACT = 22,   // count of the pit fill's compacted fill list

@@ -1,11 +1,12 @@
-// Tile worklists for the iterative stencil stages (pit fill, certification,
-// flat resolution).  In a pass, each listed 64x64 tile is taken by one
-// 256-thread workgroup of the persistent kernel; the tile iterates to a local
-// fixed point in LDS against the halo it loaded, writes back, and lists the
-// neighbour tiles whose halo it changed (border cells only) for the next
-// pass.  A per-tile epoch stamp de-duplicates the next list without clearing
-// it.  The passes stop when one lists nothing: then every tile is at a fixed
-// point with respect to its neighbours' final values.
+// Tiles of the iterative stencil stages: row solves of a tile in LDS (both pit
+// fills), and tile worklists (flat resolution, pit fill by rounds).  In a
+// pass, each listed 64x64 tile is taken by one 256-thread workgroup of the
+// persistent kernel; the tile iterates to a local fixed point in LDS against
+// the halo it loaded, writes back, and lists the neighbour tiles whose halo
+// it changed (border cells only) for the next pass.  A per-tile epoch stamp
+// de-duplicates the next list without clearing it.  The passes stop when one
+// lists nothing: then every tile is at a fixed point with respect to its
+// neighbours' final values.
 #pragma once
 
 #include "common.hpp"
@@ -200,8 +201,8 @@ __device__ inline void scan_clamp_down(float& lo, float& hi, ClampCarry& c) {
 // sweep.  The sweeps take the strip index through readfirstlane: the
 // compiler cannot tell that threadIdx.x >> 6 is the same across a wave, and
 // would otherwise keep this word, the row index and every test on them in
-// vector registers behind divergent branches (the pit fill's persistent
-// kernel: 168 VGPRs and a spill before, 106 and none after; 4.8 -> 4.6 ms).
+// vector registers behind divergent branches (the persistent kernel of the pit
+// fill by rounds: 168 VGPRs and a spill before, 106 and none after; 4.8 -> 4.6 ms).
 static_assert(STRIP == 16, "two strip masks share a word");
 __device__ inline uint32_t strip_rows(unsigned long long dirty, int strip) {
     const uint32_t m = (uint32_t)(dirty >> (strip * STRIP)) & 0xffffu;

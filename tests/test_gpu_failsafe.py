@@ -1,8 +1,9 @@
-"""Fail-safe grid barrier of the persistent kernels, forced from the host.
+"""Fail-safe waits of the persistent kernels, forced from the host.
 
-The persistent kernels (pit fill, flow routing, flow tracing) wait at grid
-barriers.  Each wait is bounded and also ends when the host raises the
-context's abort word; then every workgroup leaves normally and the call
+The flow routing waits at grid barriers and the pit fill for the tiles of
+other workgroups.  Each wait is bounded and also ends when the host raises the
+context's abort word, which the flow tracing reads at its start; then every
+workgroup leaves normally and the call
 returns CAGEO_ERR_ABORTED (-7).  These tests force both conditions from the
 host (the abort word raised before the call; a wait bound of zero), so every
 kernel still exits normally, and then check that the same context, cleared,
