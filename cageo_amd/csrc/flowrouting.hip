@@ -244,7 +244,7 @@ __device__ inline void ring_offers(Levels& v, const int* d) {
 // (A front along a row meets 64 of them in one lane: such rows are compared by
 // the whole wave.  With all of them cell by cell, a wide flat whose tiles the
 // distances cross more than once, a constant 1100 x 1100, took 1549 us to
-// route, 503 now.)
+// route, 489 now.)
 // A chain of levels, each about 100 vector instructions of one wave, bounds
 // it; the step numbers are recorded in bit planes because a store a cell
 // would cost the fullest row's cells one after the other.  Sweeps of row
@@ -291,18 +291,21 @@ __device__ inline void flat_levels(Levels& v, FrTile& T, FrSolve& S) {
         Row64 old = c & v.fin;
         v.inf &= ~set;
         v.fin &= ~old;
-        constexpr int OLD_FEW = 4;  // of a row: compared cell by cell
-        for (Row64 many = __ballot(__popcll(old) > OLD_FEW); many != 0; many &= many - 1) {
-            const int r = __builtin_ctzll(many);
-            const Row64 better = __ballot(T.d[(r + 1) * HALO_W + lane + 1] > v.level) & row_read(old, r);
-            row_write(set, set | better, r);
-            row_write(old, 0ull, r);
-        }
-        while (__ballot(old != 0)) {
-            if (old != 0) {
-                const int x = __builtin_ctzll(old);
-                old &= old - 1;
-                if (T.d[(lane + 1) * HALO_W + x + 1] > v.level) set |= 1ull << x;
+        if (__ballot(old != 0)) {
+            constexpr int OLD_FEW = 4;  // of a row: compared cell by cell
+            for (Row64 many = __ballot(__popcll(old) > OLD_FEW); many != 0; many &= many - 1) {
+                const int r = __builtin_ctzll(many);
+                const Row64 better =
+                    __ballot(T.d[(r + 1) * HALO_W + lane + 1] > v.level) & row_read(old, r);
+                row_write(set, set | better, r);
+                row_write(old, 0ull, r);
+            }
+            while (__ballot(old != 0)) {
+                if (old != 0) {
+                    const int x = __builtin_ctzll(old);
+                    old &= old - 1;
+                    if (T.d[(lane + 1) * HALO_W + x + 1] > v.level) set |= 1ull << x;
+                }
             }
         }
         v.front = set;
