@@ -468,9 +468,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
 // there and those of the three after it are on their way from memory.
 // ROWS rows x 64 pixels a workgroup, ROWS x CW waves, each a row and 16 NT
 // output channels.
-// Bound by the LDS reads of a step and the barrier that ends it (384 cycles of
-// reads for 256 of products with eight waves); the pixels take the LDS of one
-// such workgroup a CU, so eight waves are better than four that reuse more
+// Bound by the LDS reads of a step (384 cycles for 256 of products with eight
+// waves) and their latency; a barrier every three steps instead of one each
+// gained 1 %.  The pixels often take the LDS of one workgroup a CU, so eight
+// waves are better than four that reuse more
 // (384 -> 128 channels upsampled at 252 x 176: 82 us against 101), and staging
 // an upsampled input at full size took 120.  A 1001 x 700 prediction takes
 // 0.52 ms; with k_conv3x3 in its place 1.18, with the staged kernel's order
