@@ -471,9 +471,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
 // Bound by the LDS reads of a step (384 cycles for 256 of products with eight
 // waves) and their latency; a barrier every three steps instead of one each
 // gained 1 %.  The pixels often take the LDS of one workgroup a CU, so eight
-// waves are better than four that reuse more
-// (384 -> 128 channels upsampled at 252 x 176: 82 us against 101), and staging
-// an upsampled input at full size took 120.  A 1001 x 700 prediction takes
+// waves are better than four that reuse more (384 -> 128 channels upsampled
+// at 252 x 176: 82 us against 101; with the upsampled input staged at full
+// size, which leaves room for one row, 186).  A 1001 x 700 prediction takes
 // 0.52 ms; with k_conv3x3 in its place 1.18, with the staged kernel's order
 // 0.44.
 constexpr int CT_LDS = 160 * 1024;
